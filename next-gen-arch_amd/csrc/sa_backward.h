@@ -39,19 +39,16 @@ struct BwdParams {
   // Σ O''_{t,j} ⊙ dout_{t,h} (O''_{t,j} = Σ_k P_{t,j,k} v2_k), [hk * hsub]
   // [qblocks][nr][31 + NQ][DV]; null: the dk1 / dv1 pass computes dv1
   float* dv1p;
-  // Short windows of 65-128 keys (33-64 at score width 256): the dk2 / dv2
-  // passes run as two launches and carry the first one's fp32 sums here,
-  // [tokens][hk][D] then [tokens][hk][DV]; null: the portable dk2 / dv2 pass
-  float* dkv2p;
   // fp32 inputs on the matrix cores: k2 and v2 as rows of [hi: D | lo: D]
   // bf16 terms ([tokens][hk][2 D], split_hilo in the workspace); q, k1, v1,
   // dout stay fp32 and their products are split in the kernels
   const bf16* k2s;
   const bf16* v2s;
   int f32;
-  // dk2 / dv2 walk splits (bwd_dkv2_plan): each split's fp32 sums over its
-  // part of the queries reaching a key, [splits][tokens][hk][max(D, DV)],
-  // added in split order by a second kernel; null with one split
+  // dk2 / dv2 walk pieces: each piece's fp32 sums over its part of the queries
+  // reaching a key, [pieces][tokens][hk][D + DV] (dk2, then dv2), added in
+  // piece order by a second kernel.  The space of the dk1 / dv1 partials, free
+  // again by then; null without scratch (one piece)
   float* dkv2s;
 };
 
@@ -64,7 +61,8 @@ inline int dq_queries_per_block(int group) { return group % 4 == 0 ? 1 : group %
 // portable pass runs instead.
 hipError_t launch_bwd_dq_mfma(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dkv1_mfma(const BwdParams& p, hipStream_t stream);
-hipError_t launch_bwd_dkv2_mfma(const BwdParams& p, hipStream_t stream);
+// scratch_bytes: the space at p.dkv2s
+hipError_t launch_bwd_dkv2_mfma(const BwdParams& p, size_t scratch_bytes, hipStream_t stream);
 // The dq pass can produce dk1 (p.dk1p set): the MFMA passes apply and the
 // short window fits two 32-row groups (one for fp32 inputs).  The MFMA dkv1
 // launch then computes dv1 only.
@@ -74,14 +72,10 @@ hipError_t launch_bwd_dk1_sum(const BwdParams& p, hipStream_t stream);
 // dv1 = the same sum of the dq pass's dv1 partials (p.dv1p, fp32 inputs)
 hipError_t launch_bwd_dv1_sum(const BwdParams& p, hipStream_t stream);
 
-// MFMA dk2 / dv2 pass: waves per workgroup (32 long keys each) and walk
-// splits (pieces of each workgroup's walk over the queries, for shapes whose
-// (key block, KV head) workgroups leave CUs idle).  A function of the shape
-// and the device's CU count only, so that the workspace query and the launch
-// agree.
-struct Dkv2Plan {
-  int nwk, splits;
-};
-Dkv2Plan bwd_dkv2_plan(int tokens, int hk, int d, int dv, int ws, int wl, bool f32, int cus);
+// The call's widths, strides and alignment fit the MFMA passes.
+bool bwd_mfma_ok(const BwdParams& p);
+
+// fp32 sums of one walk piece of the dk2 / dv2 pass
+int64_t dkv2_piece_bytes(int tokens, int hk, int d, int dv);
 
 }  // namespace sa

@@ -25,6 +25,8 @@
 //   bwd_dkv2_kernel  one workgroup per (tile of long keys, KV head) -> dk2, dv2
 // Each recomputes P from the saved LSE.  These are portable fp32-arithmetic
 // kernels (any D in {16..512}, DV in {16..256}); they are not MFMA-tiled.
+#include <algorithm>
+
 #include "sa_generic.h"
 #include "sa_launch.h"
 #include "sa_backward.h"
@@ -585,10 +587,11 @@ static size_t dv1_partial_bytes(const sa_prefill_bwd_args* a) {
   const size_t v = (qblocks * heads * nr * (31 + nq) * f.value_dim * sizeof(float) + 255) & ~(size_t)255;
   return k + v <= kDk1PartialCap ? v : 0;
 }
-// Short windows past what one MFMA dk2 / dv2 launch holds (64 keys at widths
-// <= 128, 32 at score width 256) and up to twice that: the first launch's fp32
-// dk2 and dv2 sums.
-static size_t dkv2_partial_bytes(const sa_prefill_bwd_args* a) {
+// Scratch for the walk pieces of the dk2 / dv2 pass, beside the partials above
+// (whose space the pieces also take, once they are summed).  Two rules of
+// thumb of the shape: room for the sums of a second row-group's worth of
+// queries where the short window is long for the widths, ...
+static size_t dkv2_long_bytes(const sa_prefill_bwd_args* a) {
   const sa_prefill_args& f = a->fwd;
   const bool narrow = (f.head_dim == 64 || f.head_dim == 128) && (f.value_dim == 64 || f.value_dim == 128);
   const bool wide = f.head_dim == 256 && (f.value_dim == 128 || f.value_dim == 256);
@@ -598,28 +601,37 @@ static size_t dkv2_partial_bytes(const sa_prefill_bwd_args* a) {
     return 0;
   return ((size_t)f.total_tokens * f.heads_kv * (f.head_dim + f.value_dim) * sizeof(float) + 255) & ~(size_t)255;
 }
-// bf16 dk2 / dv2 on the matrix cores in one launch (widths 64 / 128, short
-// window <= 64) whose plan cuts the walks into pieces: the pieces' fp32 sums,
-// [splits][tokens][hk][max(D, DV)] (dk2's, then, reused, dv2's)
+// ... and, at widths 64 / 128 with short windows of at most 64 keys, up to
+// eight sums of max(D, DV) where 128-key (256-key, widths of 128 that fill the
+// CUs with them) blocks leave the CUs' two workgroup slots empty.
 static size_t dkv2_split_bytes(const sa_prefill_bwd_args* a) {
   const sa_prefill_args& f = a->fwd;
-  const bool narrow = (f.head_dim == 64 || f.head_dim == 128) && (f.value_dim == 64 || f.value_dim == 128);
+  const int d = f.head_dim, dv = f.value_dim, cus = device_cu_count();
+  const bool narrow = (d == 64 || d == 128) && (dv == 64 || dv == 128);
   if (f.dtype != SA_DTYPE_BF16 || (f.flags & SA_FLAG_FORCE_GENERIC) || !narrow || f.short_window > 64 ||
-      f.heads_kv <= 0)
+      f.heads_kv <= 0 || f.total_tokens <= 0)
     return 0;
-  const Dkv2Plan pl = bwd_dkv2_plan(f.total_tokens, f.heads_kv, f.head_dim, f.value_dim, f.short_window,
-                                    f.long_window, false, device_cu_count());
-  if (pl.splits <= 1) return 0;
-  const size_t w = (size_t)(f.head_dim > f.value_dim ? f.head_dim : f.value_dim);
-  return ((size_t)pl.splits * f.total_tokens * f.heads_kv * w * sizeof(float) + 255) & ~(size_t)255;
+  const int64_t nr = f.short_window <= 32 ? 1 : 2;
+  const int64_t blocks8 = ((int64_t)f.total_tokens + 255) / 256 * f.heads_kv;
+  if (d == 128 && dv == 128 && blocks8 >= (nr == 1 ? 2 : 1) * (int64_t)cus) return 0;
+  const int64_t blocks = ((int64_t)f.total_tokens + 127) / 128 * f.heads_kv;
+  const int64_t row = 2 * (d + dv);
+  const int64_t lds = 2 * nr * 32 * (row + 64) + 64 * nr * row + 3 * ((2 * row + 1023) / 1024 * 1024) + 4096;
+  const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(160 * 1024 / lds, 2));
+  int64_t splits = std::min<int64_t>((cus * per_cu + blocks - 1) / blocks, 8);
+  splits = std::min<int64_t>(splits, ((int64_t)128 + f.long_window - 1) / 128);
+  if (splits <= 1) return 0;
+  return ((size_t)splits * f.total_tokens * f.heads_kv * std::max(d, dv) * sizeof(float) + 255) & ~(size_t)255;
 }
+// The workspace: delta and dlse rows, the hi/lo rows of fp32 inputs, then the
+// scratch (dk1 and dv1 partials, reused by the dk2 / dv2 pieces).
+static size_t bwd_scratch_offset(const sa_prefill_bwd_args* a) { return 2 * bwd_row_bytes(a) + 2 * f32_split_bytes(a); }
 size_t prefill_bwd_workspace_bytes(const sa_prefill_bwd_args* a) {
-  return 2 * bwd_row_bytes(a) + dk1_partial_bytes(a) + dkv2_partial_bytes(a) + 2 * f32_split_bytes(a) +
-         dkv2_split_bytes(a) + dv1_partial_bytes(a);
+  return bwd_scratch_offset(a) + dk1_partial_bytes(a) + dv1_partial_bytes(a) + dkv2_long_bytes(a) + dkv2_split_bytes(a);
 }
 
 template <typename T>
-static hipError_t launch_bwd_t(const BwdParams& p, hipStream_t stream) {
+static hipError_t launch_bwd_t(const BwdParams& p, size_t scratch_bytes, hipStream_t stream) {
   const int64_t nth = (int64_t)p.tokens * p.hq;
   constexpr int kRowsPerBlock = kBwdThreads / 16;
   hipLaunchKernelGGL(bwd_delta_kernel<T>, dim3((unsigned)((nth + kRowsPerBlock - 1) / kRowsPerBlock)),
@@ -661,7 +673,7 @@ static hipError_t launch_bwd_t(const BwdParams& p, hipStream_t stream) {
     }
   }
   if (e != hipSuccess) return e;
-  e = launch_bwd_dkv2_mfma(p, stream);
+  e = launch_bwd_dkv2_mfma(p, scratch_bytes, stream);
   if (e == hipErrorNotSupported) {
     hipLaunchKernelGGL(bwd_dkv2_kernel<T>, ks[2].grid, dim3(kBwdThreads), ks[2].lds, stream, p);
     e = hipGetLastError();
@@ -723,7 +735,7 @@ hipError_t launch_prefill_bwd(const sa_prefill_bwd_args* a, void* ws, hipStream_
   p.mfma = (f.dtype == SA_DTYPE_BF16 && !(f.flags & SA_FLAG_FORCE_GENERIC)) || f32_mfma_shape(f);
   if (size_t sb = f32_split_bytes(a)) {
     // k2 and v2 as hi/lo bf16 rows for the fp32 matrix-core passes
-    char* base = (char*)ws + 2 * bwd_row_bytes(a) + dk1_partial_bytes(a) + dkv2_partial_bytes(a);
+    char* base = (char*)ws + 2 * bwd_row_bytes(a);
     bf16* k2s = (bf16*)base;
     bf16* v2s = (bf16*)(base + sb);
     hipError_t e = launch_split_hilo((const float*)f.k2, f.k_stride_t, f.k_stride_h, f.total_tokens, f.heads_kv,
@@ -735,16 +747,13 @@ hipError_t launch_prefill_bwd(const sa_prefill_bwd_args* a, void* ws, hipStream_
     p.k2s = k2s;
     p.v2s = v2s;
   }
-  if (dk1_partial_bytes(a) && bwd_dk1_fused_ok(p)) p.dk1p = (float*)((char*)ws + 2 * bwd_row_bytes(a));
-  if (dv1_partial_bytes(a) && p.dk1p)
-    p.dv1p = (float*)((char*)ws + 2 * bwd_row_bytes(a) + dk1_partial_bytes(a) + dkv2_partial_bytes(a) +
-                      2 * f32_split_bytes(a) + dkv2_split_bytes(a));
-  if (dkv2_partial_bytes(a)) p.dkv2p = (float*)((char*)ws + 2 * bwd_row_bytes(a) + dk1_partial_bytes(a));
-  if (dkv2_split_bytes(a))
-    p.dkv2s = (float*)((char*)ws + 2 * bwd_row_bytes(a) + dk1_partial_bytes(a) + dkv2_partial_bytes(a) +
-                       2 * f32_split_bytes(a));
-  if (f.dtype == SA_DTYPE_F32) return launch_bwd_t<float>(p, stream);
-  return launch_bwd_t<bf16>(p, stream);
+  char* const scratch = (char*)ws + bwd_scratch_offset(a);
+  const size_t scratch_bytes = prefill_bwd_workspace_bytes(a) - bwd_scratch_offset(a);
+  if (dk1_partial_bytes(a) && bwd_dk1_fused_ok(p)) p.dk1p = (float*)scratch;
+  if (dv1_partial_bytes(a) && p.dk1p) p.dv1p = (float*)(scratch + dk1_partial_bytes(a));
+  if (scratch_bytes) p.dkv2s = (float*)scratch;
+  if (f.dtype == SA_DTYPE_F32) return launch_bwd_t<float>(p, scratch_bytes, stream);
+  return launch_bwd_t<bf16>(p, scratch_bytes, stream);
 }
 
 }  // namespace sa

@@ -22,11 +22,7 @@
 //     S^T, dP^T, dS as above (A rows q_t ⊙ k1_j, B rows dout_t ⊙ v1_j)
 //     G^T  += K2^T · dS^T,  O''^T += V2^T · bf16(P)^T     (d x t)
 //     dk1_j = Σ_h Σ_t G_t ⊙ q_t,   dv1_j = Σ_h Σ_t O''_t ⊙ dout_t
-//   dk2/dv2 pass (one wave per 32 long keys, their K2/V2 rows held as MFMA
-//   fragments; the workgroup streams every (t, h) that reaches its keys and
-//   builds that step's A_t / B_t rows (32 short keys j) in LDS)
-//     S^T = A_t · K2^T, dP^T = B_t · V2^T                (j x keys)
-//     dK2^T += A_t^T · dS^T,  dV2^T += B_t^T · bf16(P)^T  (d x keys)
+//   dk2/dv2 pass: sa_backward_dkv2.hip
 //
 // The tile machinery (LDS ring filled by global->LDS DMA, TileGeom layouts,
 // the transposing-read accumulation) is the forward kernel's (sa_mfma.h).
@@ -41,14 +37,10 @@ namespace {
 // LDS fragments read ahead of their MFMA in each pass (see BwdOps; dq two
 // ahead at widths up to 128: NS forward + backward 17.05 -> 16.96 ms, the
 // adapter shape 8.85 -> 8.74 ms); at score width 256 (one wave per SIMD: no
-// other wave hides the LDS latency) the dq and dk2 / dv2 passes read further
-// ahead (C4 forward + backward 29.1 -> 28.7 and 28.9 ms)
+// other wave hides the LDS latency) the dq pass reads further ahead (C4
+// forward + backward 29.1 -> 28.7 ms)
 constexpr int kDqPF = 2, kDqPFWide = 3;      // dq pass
 constexpr int kDk1PF = 1;                    // dk1 / dv1 pass (dv1 reads two ahead)
-constexpr int kDkv2PF = 2, kDkv2PFWide = 4;  // dk2 / dv2 pass
-
-constexpr size_t kLdsPerCu = 160 * 1024;  // gfx950
-constexpr int kMaxWalkSplits = 8;         // dk2 / dv2 walk pieces per (key block, KV head)
 
 // Wave-level tile products used by the backward passes (D = head dim).
 template <int D>
@@ -1196,685 +1188,6 @@ __global__ __launch_bounds__(256) void bwd_dk1_sum_kernel(BwdParams p, int qbloc
 }
 
 
-// ---------------------------------------------------------------------------
-// dk2, dv2: a workgroup of NWK waves owns 32 * NWK consecutive long keys of
-// one KV group; wave w's 32 keys are kw = k0 + 32w + lane % 32.  It walks the
-// steps (t, h) for t = k0 .. k0 + 32 NWK - 1 + wl - 1 (every query whose long
-// window can reach a key of the block) and h over the group's heads.  Per
-// step the waves build, per 32-row group r < NR of short keys, A_t (rows
-// j = t - 32r - 31 .. t - 32r: bf16(q_th ⊙ k1_j)) and B_t (bf16(dout_th ⊙
-// v1_j)) in LDS, 32 / NWK rows each; tiles are double-buffered, one barrier
-// per step.  Wider blocks (NWK = 8 at D = 128) share each step's tile
-// formation, barrier and staging among more keys.  The last wave stages each
-// step's q, dout, k1_t and v1_t rows with one full-wave DMA two steps ahead; the
-// k1 / v1 rows of earlier queries come from a 64·NR-row ring (row j at slot
-// j % (64 NR)) into which wave 0 copies each staged k1_t / v1_t.  Covers
-// ws <= 32 NR (NR = 1, 2).
-
-// MODE 1: dK2 only, MODE 2: dV2 only (two launches).  Each holds one
-// accumulator set, and the dV2 launch neither the V2 fragments nor dP, so
-// both fit two waves per SIMD; the S recomputation is paid twice.
-// MODE 3 (fp32 inputs, which run one wave per SIMD either way): dK2 and dV2
-// in one launch from one S per step and one formation of the A / B rows.
-// PH (phased): twice the short-key rows of one launch run as two launches,
-// phase 1 (row groups 0 .. NR-1: rows j = t - 32 NR + 1 .. t) writing its fp32
-// sums to p.dkv2p and phase 2 (groups NR .. 2NR-1) starting from them and
-// writing the gradient; widths of 256 (one group per launch) always run so.
-// Without PH, phase is 0 (one launch).
-// F32: fp32 inputs (DK == DV <= 128, NR = 1): the K2 / V2 fragments from the
-// hi/lo rows (hi and lo fragments), fp32 q / dout / k1 / v1 rows in the
-// stage and the ring, A / B tile rows formed as [hi: D | lo: D] from fp32
-// products, three term pairs per product, fp32 output.
-// splits > 1 (one launch, bf16): the workgroups of a (key block, KV head)
-// walk contiguous pieces of its queries and write fp32 sums to p.dkv2s
-// ([split][tokens][hk][XW]); bwd_dkv2_sum_kernel adds them in split order.
-template <int DK, int DV, int MODE, int NWK, int NR, bool PH, bool F32 = false>
-__global__ __launch_bounds__(64 * NWK, (DK > 128 || F32) ? 1 : 2) void bwd_dkv2_mfma_kernel(BwdParams p,
-                                                                                           int nblocks, int phase,
-                                                                                           int splits) {
-  static_assert(!F32 || (DK == DV && DK <= 128 && NR == 1 && !PH), "fp32 inputs: equal widths up to 128, one group");
-  constexpr bool kBoth = MODE == 3;  // dK2 and dV2 (fp32)
-  static_assert(!kBoth || F32, "both gradients in one launch: fp32 inputs");
-  constexpr bool kDK = MODE == 1 || kBoth, kDV = MODE == 2 || kBoth;
-  constexpr int EW = F32 ? 2 : 1;  // bf16 units per element of an LDS row
-  constexpr int kKvRing = 64 * NR;  // k1 / v1 ring rows (a power of two)
-  constexpr int KB = 32 * NWK;    // keys per workgroup
-  constexpr int RPW = 32 / NWK;   // A / B rows formed per wave and step
-  // LDS reads in flight ahead of their MFMA: with two waves per SIMD, one
-  // read ahead leaves each step's three MFMA chains waiting on LDS latency
-  constexpr int kPF = DK >= 256 ? kDkv2PFWide : kDkv2PF;
-  static_assert(kDK || kDV, "an output per launch");
-  constexpr int XW = kDK ? DK : DV;        // width of the gradient accumulated in acc (dK2 when both)
-  using OPK = BwdOps<DK>;
-  using OPV = BwdOps<DV>;
-  // A / B tile row strides (padded: row and transposing reads)
-  constexpr int RSA = 2 * EW * DK + 32, RSB = 2 * EW * DV + 32;
-  constexpr int TA = 32 * RSA, TAB = TA + 32 * RSB;  // one A tile, one A + B pair
-  constexpr int RBK = 2 * EW * DK, RBV = 2 * EW * DV;  // k1 / v1 row bytes (q / dout rows alike)
-  constexpr int RKV = RBK + RBV;             // ring row: k1 then v1
-  constexpr int SS = (2 * RKV + 1023) / 1024 * 1024, SI = SS / 1024;  // stage slot bytes, DMA instructions
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  char* const tiles = lds;                        // [2 buffers][NR groups][A, B]
-  char* const ring = tiles + 2 * NR * TAB;        // [64 NR slots][k1 row, v1 row]
-  char* const stage = ring + kKvRing * RKV;       // [3][q row, dout row, k1_t row, v1_t row] (SS bytes each)
-
-  const int tid = tid_x(), lane = tid & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int half = lane >> 5, n = lane & 31;
-  // per wave: the per-step scalars of 64 steps, 16 bytes each
-  floatx4* const scal = (floatx4*)(stage + 3 * SS) + 64 * wid;
-  constexpr bool kPhased = PH;
-  const int r0 = kPhased && phase == 2 ? NR : 0;  // row group offset of this launch (the ring holds 64 NR rows)
-  // walk splits: bf16 single launches only (the launcher passes 1 otherwise)
-  constexpr bool kSplit = !PH && !F32;
-  const int nsplit = kSplit ? splits : 1;
-  const int lb = xcd_remap(bid_x(), nblocks);
-  const int kblocks = (p.tokens + KB - 1) / KB;
-  const int kb = lb % kblocks;
-  const int g = kSplit ? lb / kblocks % p.hk : lb / kblocks;
-  const int split = kSplit ? lb / kblocks / p.hk : 0;
-  const int k0 = kb * KB;
-  const int last = p.tokens - 1;
-  const int kw = k0 + 32 * wid + n;  // this lane's key (column of the C layout)
-  const int kwc = min(kw, last);
-  const bool kvalid = kw < p.tokens;
-  const int G = p.group;
-  const int64_t kvg_k = (int64_t)g * p.k_sh, kvg_v = (int64_t)g * p.v_sh;
-
-  // K2 / V2 rows of the wave's keys as B operands (k = d): lane (n, half)
-  // holds d = 16t + 8*half .. +7 of key kw.
-  // (fp32: the hi/lo rows [tokens][hk][2 D], hi fragments in kf / vf, lo in kfl / vfl)
-  const bf16* k2r = F32 ? p.k2s + ((int64_t)kwc * p.hk + g) * 2 * DK : (const bf16*)p.k2 + (int64_t)kwc * p.k_st + kvg_k;
-  const bf16* v2r = F32 ? p.v2s + ((int64_t)kwc * p.hk + g) * 2 * DV : (const bf16*)p.v2 + (int64_t)kwc * p.v_st + kvg_v;
-  bf16x8 kf[DK / 16], vf[kDK ? DV / 16 : 1];
-  bf16x8 kfl[F32 ? DK / 16 : 1], vfl[F32 && kDK ? DV / 16 : 1];
-#pragma unroll
-  for (int t = 0; t < DK / 16; ++t) {
-    kf[t] = *(const bf16x8*)(k2r + 16 * t + 8 * half);
-    if constexpr (F32) kfl[t] = *(const bf16x8*)(k2r + DK + 16 * t + 8 * half);
-  }
-  if constexpr (kDK) {
-#pragma unroll
-    for (int t = 0; t < DV / 16; ++t) {
-      vf[t] = *(const bf16x8*)(v2r + 16 * t + 8 * half);
-      if constexpr (F32) vfl[t] = *(const bf16x8*)(v2r + DV + 16 * t + 8 * half);
-    }
-  }
-  floatx16 acc[XW / 32];  // dK2^T or dV2^T
-#pragma unroll
-  for (int i = 0; i < XW / 32; ++i) acc[i] = floatx16{};
-  floatx16 accv[kBoth ? DV / 32 : 1];  // dV2^T (both gradients)
-#pragma unroll
-  for (int i = 0; i < (kBoth ? DV / 32 : 1); ++i) accv[i] = floatx16{};
-  // fp32 sums of the first row group (phases 1 and 2): [tokens][hk][DK] for
-  // dK2, then [tokens][hk][DV] for dV2, each lane's values at its d
-  auto part_row = [&]() {
-    return p.dkv2p + (kDK ? 0 : (int64_t)p.tokens * p.hk * DK) + ((int64_t)kwc * p.hk + g) * XW;
-  };
-  if (kPhased && phase == 2 && kvalid) {
-    const float* part = part_row();
-#pragma unroll
-    for (int db = 0; db < XW / 32; ++db)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const floatx4 x = *(const floatx4*)(part + 32 * db + 8 * q4 + 4 * half);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[db][4 * q4 + e] = x[e];
-      }
-  }
-
-  // the queries reaching the block's keys, t = k0 .. min(last, k0 + KB + wl - 2),
-  // cut into `splits` contiguous pieces; this workgroup walks piece `split`
-  const int walk = min(last, k0 + KB - 1 + p.wl - 1) - k0 + 1;
-  const int tfirst = k0 + (int)((int64_t)walk * split / nsplit);
-  const int tlast = k0 + (int)((int64_t)walk * (split + 1) / nsplit) - 1;
-  // step s <-> (t = tfirst + s / G, h = g*G + s % G)
-  const int nsteps = (tlast - tfirst + 1) * G;
-  // write: acc[db] holds d = 32*db + acc_row(r, half) of key kw
-  auto write_out = [&]() {
-    if (!kvalid) return;
-    if (kSplit && nsplit > 1) {
-      float* part = p.dkv2s + (((int64_t)split * p.tokens + kw) * p.hk + g) * XW;
-#pragma unroll
-      for (int db = 0; db < XW / 32; ++db)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          floatx4 x;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x[e] = acc[db][4 * q4 + e];
-          *(floatx4*)(part + 32 * db + 8 * q4 + 4 * half) = x;
-        }
-    } else if (kPhased && phase == 1) {
-      float* part = part_row();
-#pragma unroll
-      for (int db = 0; db < XW / 32; ++db)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          floatx4 x;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x[e] = acc[db][4 * q4 + e];
-          *(floatx4*)(part + 32 * db + 8 * q4 + 4 * half) = x;
-        }
-    } else if (F32) {
-      // key and half from a fresh lane id: row addresses formed here, not
-      // held (or spilled) through the step loop
-      const int lf = fresh_lane();
-      const int kwf = k0 + 32 * wid + (lf & 31), hf = lf >> 5;
-      float* orow = kDK ? (float*)p.dk2 + (int64_t)kwf * p.dk_st + (int64_t)g * p.dk_sh
-                        : (float*)p.dv2 + (int64_t)kwf * p.dv_st + (int64_t)g * p.dv_sh;
-#pragma unroll
-      for (int db = 0; db < XW / 32; ++db)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          floatx4 a;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a[e] = acc[db][4 * q4 + e];
-          *(floatx4*)(orow + 32 * db + 8 * q4 + 4 * hf) = a;
-        }
-      if constexpr (kBoth) {
-        float* vrow = (float*)p.dv2 + (int64_t)kwf * p.dv_st + (int64_t)g * p.dv_sh;
-#pragma unroll
-        for (int db = 0; db < DV / 32; ++db)
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            floatx4 a;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a[e] = accv[db][4 * q4 + e];
-            *(floatx4*)(vrow + 32 * db + 8 * q4 + 4 * hf) = a;
-          }
-      }
-    } else {
-      bf16* orow = kDK ? (bf16*)p.dk2 + (int64_t)kw * p.dk_st + (int64_t)g * p.dk_sh
-                       : (bf16*)p.dv2 + (int64_t)kw * p.dv_st + (int64_t)g * p.dv_sh;
-#pragma unroll
-      for (int db = 0; db < XW / 32; ++db)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const int d = 32 * db + 8 * q4 + 4 * half;
-          bf16x4 a;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a[e] = (bf16)acc[db][4 * q4 + e];
-          *(bf16x4*)(orow + d) = a;
-        }
-    }
-  };
-  // an empty piece (a short last key block): zero sums (uniform, before any
-  // barrier); one piece always holds t = k0
-  if (kSplit && nsteps <= 0) {
-    write_out();
-    return;
-  }
-
-  // Step st <-> (t = tfirst + st / G, h = g*G + st % G), stage slot st % 3:
-  // carried from step to step (no divisions in the step loop).
-  struct Step {
-    int t, h, slot;
-  };
-  auto advance = [&](Step x) {
-    Step y{x.t, x.h + 1, x.slot == 2 ? 0 : x.slot + 1};
-    if (y.h == g * G + G) y.h = g * G, ++y.t;
-    return y;
-  };
-  // The staging wave stages step st: lane -> byte 16 lane of the rows q,
-  // dout, k1_t, v1_t laid end to end (lanes past them re-fetch the q row's
-  // first segment into the unused tail); every lane active, one instruction
-  // per 1 KB.  Every wave waits for the staging wave at the step's barrier, so
-  // its addresses are selected per lane without branches (a lane's tensor is
-  // fixed by its byte offset b), the row offsets formed once per step in
-  // scalars.  Four-wave workgroups stage from the last wave (wave 0 copies
-  // rows into the ring): dk2 / dv2 3-4 % faster at the adapter shape and at
-  // width 256 than from wave 0; eight-wave ones from wave 0 (the last wave
-  // measured 4 % slower there).
-  constexpr int kDmaWave = NWK >= 8 ? 0 : NWK - 1;
-  auto dma_step = [&](int st, Step x) {
-    if (wid != kDmaWave || st >= nsteps) return;
-    // element offsets of the step's rows (uniform)
-    const int64_t oq = (int64_t)x.t * p.q_st + (int64_t)x.h * p.q_sh;
-    const int64_t og = (int64_t)x.t * p.do_st + (int64_t)x.h * p.do_sh;
-    const int64_t ok = (int64_t)x.t * p.k_st + kvg_k, ov = (int64_t)x.t * p.v_st + kvg_v;
-#pragma unroll
-    for (int k = 0; k < SI; ++k) {
-      // byte offset from a fresh lane id: not hoisted into registers held through the step loop
-      int b = 1024 * k + 16 * fresh_lane();
-      if (b >= 2 * RKV) b = 0;
-      const bool isq = b < RBK, isg = b < RKV, isk = b < RKV + RBK;
-      const bf16* base = isq ? (const bf16*)p.q : isg ? (const bf16*)p.dout : isk ? (const bf16*)p.k1 : (const bf16*)p.v1;
-      const int64_t oe = isq ? oq : isg ? og : isk ? ok : ov;
-      const int inrow = b - (isq ? 0 : isg ? RBK : isk ? RKV : RKV + RBK);  // bytes
-      // (element offsets scaled by EW: fp32 rows viewed as bf16 units)
-      dma16(base + EW * oe + inrow / 2, stage + x.slot * SS + 1024 * k);
-    }
-  };
-  // wave 0 copies the staged k1_t / v1_t rows of step st into ring slot t % (64 NR)
-  auto to_ring = [&](int st, Step x) {
-    if (wid != 0 || st >= nsteps) return;
-    if (lane < RKV / 16) {
-      const uint4 v = *(const uint4*)(stage + x.slot * SS + RKV + 16 * lane);
-      *(uint4*)(ring + (x.t % kKvRing) * RKV + 16 * lane) = v;
-    }
-  };
-
-  Step s_cur{tfirst, g * G, 0};
-  Step s_nx1 = advance(s_cur), s_nx2 = advance(s_nx1);
-  dma_step(0, s_cur);
-  dma_step(1, s_nx1);
-  // the k1 / v1 rows before the first query (j = tfirst - 32 NR + 1 .. tfirst - 1) into the ring
-  for (int idx = tid; idx < (32 * (NR + r0) - 1) * (RKV / 16); idx += 64 * NWK) {
-    const int jj = idx / (RKV / 16), w = idx % (RKV / 16);  // w: 16-byte segment of the ring row
-    const int j = tfirst - (32 * (NR + r0) - 1) + jj;
-    if (j >= 0) {
-      const bf16* src = w < RBK / 16 ? (const bf16*)p.k1 + EW * ((int64_t)j * p.k_st + kvg_k) + 8 * w
-                                     : (const bf16*)p.v1 + EW * ((int64_t)j * p.v_st + kvg_v) + 8 * (w - RBK / 16);
-      *(uint4*)(ring + (j % kKvRing) * RKV + 16 * w) = *(const uint4*)src;
-    }
-  }
-  wait_vmcnt<0>();
-  block_barrier();
-
-  // form A / B rows of step st into tile buffer b: wave w builds rows
-  // RPW w .. RPW w + RPW - 1 of each group; row 31 of group 0 (j = t) comes
-  // from the stage, earlier rows from the ring
-  auto form = [&](Step x, int b) {
-    const int t = x.t;
-    const char* sg_row = stage + x.slot * SS;
-    if constexpr (F32) {
-      // fp32 rows: one row and 4 elements (16 source bytes) per lane; the
-      // products q ⊙ k1 and dout ⊙ v1 split into hi (row elements 4 sg ..)
-      // and lo (elements D + 4 sg ..) bf16 terms.  A lane's 4-element group sg
-      // = lane % SEGS is the same in every row block: its q and dout values
-      // are read once, and the k1 / v1 reads of kB blocks at a time are
-      // issued before their products.
-      constexpr int SEGS = DK / 4;
-      static_assert(RPW * SEGS % 64 == 0 && 64 % SEGS == 0, "whole lanes per formed row block");
-      constexpr int NU = RPW * SEGS / 64, kB = NU < 2 ? NU : 2;
-      const int sg = lane % SEGS;
-      const floatx4 qv = *(const floatx4*)(sg_row + 16 * sg);
-      const floatx4 gv = *(const floatx4*)(sg_row + RBK + 16 * sg);
-      char* At = tiles + b * TAB;
-      char* Bt = At + TA;
-#pragma unroll
-      for (int u0 = 0; u0 < NU; u0 += kB) {
-        floatx4 kv[kB], vv[kB];
-#pragma unroll
-        for (int u = 0; u < kB; ++u) {
-          const int i = RPW * wid + ((u0 + u) * 64 + lane) / SEGS;  // tile row
-          const int j = max(t - 31 + i, 0);
-          const char* kvrow = j == t ? sg_row + RKV : ring + (j % kKvRing) * RKV;
-          kv[u] = *(const floatx4*)(kvrow + 16 * sg);
-          vv[u] = *(const floatx4*)(kvrow + RBK + 16 * sg);
-        }
-#pragma unroll
-        for (int u = 0; u < kB; ++u) {
-          const int i = RPW * wid + ((u0 + u) * 64 + lane) / SEGS;
-          bf16x4 ah, al, bh, bl;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            bf16 h_, l_;
-            split_bf16(qv[e] * kv[u][e], h_, l_);
-            ah[e] = h_;
-            al[e] = l_;
-            split_bf16(gv[e] * vv[u][e], h_, l_);
-            bh[e] = h_;
-            bl[e] = l_;
-          }
-          *(bf16x4*)(At + i * RSA + 8 * sg) = ah;
-          *(bf16x4*)(At + i * RSA + 2 * DK + 8 * sg) = al;
-          *(bf16x4*)(Bt + i * RSB + 8 * sg) = bh;
-          *(bf16x4*)(Bt + i * RSB + 2 * DV + 8 * sg) = bl;
-        }
-      }
-    } else if constexpr (DK == DV) {  // A and B rows side by side: one row and segment per lane
-      constexpr int SEGS = DK / 8;  // 16-byte segments per row
-      static_assert(RPW * SEGS % 64 == 0 && 64 % SEGS == 0, "whole lanes per formed row block");
-      constexpr int NU = NR * RPW * SEGS / 64;  // row blocks formed by each lane
-      // A lane forms segment sg = lane % SEGS of every row block, so its q and
-      // dout segments are read once; every k1 / v1 read is issued before the
-      // first product (the tile writes would otherwise keep each block's reads
-      // behind the previous block's writes: one LDS latency per block).
-      const int sg = lane % SEGS;
-      const u32x4 q4 = __builtin_bit_cast(u32x4, *(const bf16x8*)(sg_row + 16 * sg));
-      const u32x4 g4 = __builtin_bit_cast(u32x4, *(const bf16x8*)(sg_row + RBK + 16 * sg));
-      u32x4 k4[NU], v4[NU];
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const int r = u / (RPW * SEGS / 64);  // row group
-        const int i = RPW * wid + ((u % (RPW * SEGS / 64)) * 64 + lane) / SEGS;  // tile row
-        const int j = max(t - 32 * (r + r0) - 31 + i, 0);
-        const char* kvrow = j == t ? sg_row + RKV : ring + (j % kKvRing) * RKV;
-        k4[u] = __builtin_bit_cast(u32x4, *(const bf16x8*)(kvrow + 16 * sg));
-        v4[u] = __builtin_bit_cast(u32x4, *(const bf16x8*)(kvrow + RBK + 16 * sg));
-      }
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const int r = u / (RPW * SEGS / 64);
-        char* At = tiles + (b * NR + r) * TAB;
-        char* Bt = At + TA;
-        const int i = RPW * wid + ((u % (RPW * SEGS / 64)) * 64 + lane) / SEGS;
-        u32x4 a, bb;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          a[e] = mul_bf16_pair(q4[e], k4[u][e]);
-          bb[e] = mul_bf16_pair(g4[e], v4[u][e]);
-        }
-        *(u32x4*)(At + i * RSA + 16 * sg) = a;
-        *(u32x4*)(Bt + i * RSB + 16 * sg) = bb;
-      }
-    } else {  // A rows (DK / 8 segments), then B rows (DV / 8)
-      constexpr int SK = DK / 8, SV = DV / 8;
-      static_assert(RPW * SK % 64 == 0 && RPW * SV % 64 == 0 && 64 % SK == 0 && 64 % SV == 0,
-                    "whole lanes per formed row block");
-      constexpr int UA = RPW * SK / 64, UB = RPW * SV / 64, NU = NR * (UA + UB);
-      // as above: a lane's q (dout) segment lane % SK (lane % SV) is the same
-      // in every A (B) block, read once; every k1 / v1 read is issued first
-      const u32x4 q4 = __builtin_bit_cast(u32x4, *(const bf16x8*)(sg_row + 16 * (lane % SK)));
-      const u32x4 g4 = __builtin_bit_cast(u32x4, *(const bf16x8*)(sg_row + RBK + 16 * (lane % SV)));
-      u32x4 y4[NU];
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const int r = u / (UA + UB), v = u % (UA + UB);  // row group, instruction within it
-        const bool isb = v >= UA;
-        const int segs = isb ? SV : SK, off = isb ? RBK : 0;
-        const int idx = (isb ? v - UA : v) * 64 + lane;
-        const int i = RPW * wid + idx / segs, sg = idx % segs;  // tile row, segment
-        const int j = max(t - 32 * (r + r0) - 31 + i, 0);
-        const char* kvrow = j == t ? sg_row + RKV : ring + (j % kKvRing) * RKV;
-        y4[u] = __builtin_bit_cast(u32x4, *(const bf16x8*)(kvrow + off + 16 * sg));
-      }
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const int r = u / (UA + UB), v = u % (UA + UB);
-        const bool isb = v >= UA;
-        const int segs = isb ? SV : SK;
-        const int idx = (isb ? v - UA : v) * 64 + lane;
-        const int i = RPW * wid + idx / segs, sg = idx % segs;
-        const u32x4 x4 = isb ? g4 : q4;
-        u32x4 a;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) a[e] = mul_bf16_pair(x4[e], y4[u][e]);
-        char* At = tiles + (b * NR + r) * TAB;
-        *(u32x4*)(isb ? At + TA + i * RSB + 16 * sg : At + i * RSA + 16 * sg) = a;
-      }
-    }
-  };
-
-  const float sl2s = p.scale * kLog2e;
-  // Sequence of t, tracked as the start s0 of t's sequence and the first
-  // token past it (dense: a boundary every seqlen; packed: the cu walk, one
-  // load per boundary crossed).
-  int seq = 0, s0 = 0, snext = 0;
-  if (p.cu != nullptr) {
-    int lo = 0, hi = p.num_seqs - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (p.cu[mid] <= tfirst) lo = mid;
-      else hi = mid - 1;
-    }
-    seq = lo;
-    snext = tfirst;  // first step loads the start and the next boundary
-  } else {
-    s0 = (tfirst / p.seqlen) * p.seqlen;
-    snext = s0 + p.seqlen;
-  }
-  // Per-step scalars (lse, and for dK2 dl and delta of (t, h)): loaded one
-  // lane per step, 64 steps at a time and one block ahead, and kept in a
-  // wave-private LDS table, so that a step reads them from LDS instead of
-  // waiting on a global load.
-  floatx4 nx{};  // this lane's step of the next block (loads in flight)
-  auto load_block = [&](int blk) {
-    const int si = min(64 * blk + lane, nsteps - 1);
-    const int tq = tfirst + si / G, hq = g * G + si % G;
-    const int64_t thq = (int64_t)tq * p.hq + hq;
-    nx[0] = p.lse[(int64_t)tq * p.lse_st + hq];
-    if constexpr (kDK) {
-      nx[1] = p.dl[thq];
-      nx[2] = p.delta[thq];
-    }
-  };
-  auto store_block = [&]() {
-    // the wait is tied to these registers: later steps need none
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(nx));
-    scal[lane] = nx;
-  };
-  load_block(0);
-  store_block();
-  if (nsteps > 64) load_block(1);
-  to_ring(0, s_cur);
-  form(s_cur, 0);
-  for (int st = 0; st < nsteps; ++st) {
-    const int sl = st & 63;
-    if (sl == 0 && st > 0) {  // next block: its values into the table, load the one after
-      store_block();
-      if (st + 64 < nsteps) load_block((st >> 6) + 1);
-    }
-    // staging wave: the rows of step st+1 have landed (step st+2's may be in flight)
-    if (wid == kDmaWave) {
-      dma_step(st + 2, s_nx2);
-      if (st + 2 < nsteps) wait_vmcnt<SI>();
-      else wait_vmcnt<0>();
-    }
-    block_barrier();  // tiles of st formed, ring rows up to t(st) copied; rows of st+1 staged; buffer (st+1)%2 free
-    const Step s_now = s_cur, s_form = s_nx1;
-    s_cur = s_nx1, s_nx1 = s_nx2, s_nx2 = advance(s_nx2);
-
-    const int t = s_now.t;
-    if (t >= snext) {  // crossed into another sequence (uniform, rare)
-      if (p.cu == nullptr) {
-        s0 = (t / p.seqlen) * p.seqlen;
-        snext = s0 + p.seqlen;
-      } else {
-        while (seq + 1 < p.num_seqs && p.cu[seq + 1] <= t) ++seq;
-        const int c = p.cu[seq];
-        s0 = min(max(c, 0), t);
-        // well formed (cu[seq] <= t): the start holds up to the next boundary
-        snext = c > t ? t + 1 : (seq + 1 < p.num_seqs ? p.cu[seq + 1] : 0x7fffffff);
-      }
-      s0 = __builtin_amdgcn_readfirstlane(s0);
-      snext = __builtin_amdgcn_readfirstlane(snext);
-    }
-    const floatx4 sv4 = scal[sl];  // wave-private: this wave's table writes are ordered before
-    const float lse2 = sv4[0] * kLog2e;
-    const bool single = t == s0 || (p.ws == 1 && p.wl == 1);
-    const float dpm = single ? 0.f : p.scale;
-    const float dsm = kDK ? (single ? sv4[1] * p.scale : -sv4[2] * p.scale) : 0.f;
-    // validity: key kw in [max(s0, t - wl + 1), t]; row i (j = t - 31 + i) in [max(s0, t - ws + 1), t]
-    const bool kok = kvalid && kw <= t && kw >= max(s0, t - p.wl + 1);
-    const int ilo = max(s0, t - p.ws + 1) - (t - 31 - 32 * r0);
-    // a wave none of whose 32 keys lies in t's long window skips the step
-    // (about a fifth of the steps at the block's ends)
-    const int kw0 = k0 + 32 * wid;
-    const bool skip = kw0 > t || kw0 + 31 < max(s0, t - p.wl + 1) || kw0 >= p.tokens;
-    const char* At = tiles + (st & 1) * NR * TAB;  // group 0
-    const char* Bt = At + TA;
-    floatx16 sv, dp;
-    if (!skip) {
-      if constexpr (F32) {
-        sv = OPK::template rows_x_hl<RSA>(At, 0, lane, kf, kfl);  // C[j][key]
-        if constexpr (kDK) dp = OPV::template rows_x_hl<RSB>(Bt, 0, lane, vf, vfl);
-      } else {
-        sv = OPK::template rows_x<RSA, kPF>(At, 0, lane, kf);  // C[j][key]
-        if constexpr (kDK) dp = OPV::template rows_x<RSB, kPF>(Bt, 0, lane, vf);
-      }
-    }
-    // the next step's rows are formed after this step's S (and dP) MFMAs are
-    // issued: the VALU work runs while the matrix cores work (the two waves
-    // of a SIMD are in step with each other through the barrier, so their
-    // VALU phases would otherwise coincide with an idle matrix pipe)
-    if (st + 1 < nsteps) {
-      to_ring(st + 1, s_form);  // slot t(st+1) % 64 is read only from the next iteration on
-      form(s_form, (st + 1) & 1);
-    }
-    if (skip) continue;
-    // group r: the probabilities (dS or P) from its scores, then
-    // dK2^T += A_t^T · dS^T, or dV2^T += B_t^T · P^T
-    auto accumulate = [&](const floatx16& s_, const floatx16& dp_, int ilo_r, const char* At_r, const char* Bt_r) {
-      if constexpr (F32) {
-        // dS (dK2) and / or P (dV2) in fp32, as hi/lo B operands
-        float x[16], pv[kBoth ? 16 : 1];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int ie = 8 * (e >> 2) + 4 * half + (e & 3);
-          const bool ok = kok && ie >= ilo_r;
-          const float pe = ok ? fast_exp2(fmaf(s_[e], sl2s, -lse2)) : 0.f;
-          if constexpr (kDK) x[e] = pe * fmaf(dp_[e], dpm, dsm);
-          else x[e] = pe;
-          if constexpr (kBoth) pv[e] = pe;
-        }
-        bf16x8 b0, b1, l0, l1;
-        OPK::pack_c_hl(x, b0, b1, l0, l1);
-        if constexpr (kDK) OPK::template tr_acc_hl<RSA>(acc, At_r, 0, lane, b0, b1, l0, l1);
-        else OPV::template tr_acc_hl<RSB>(acc, Bt_r, 0, lane, b0, b1, l0, l1);
-        if constexpr (kBoth) {
-          OPK::pack_c_hl(pv, b0, b1, l0, l1);
-          OPV::template tr_acc_hl<RSB>(accv, Bt_r, 0, lane, b0, b1, l0, l1);
-        }
-        return;
-      }
-      uint32_t pk[8];  // bf16(dS) (dK2 launch) or bf16(P) (dV2 launch)
-      if (ilo_r <= 0) {  // every row valid (uniform test); keys outside: exp2(s*c - inf) = 0
-        const float lse2k = kok ? lse2 : INFINITY;
-#pragma unroll
-        for (int e = 0; e < 16; e += 2) {
-          const float p0 = fast_exp2(fmaf(s_[e], sl2s, -lse2k)), p1 = fast_exp2(fmaf(s_[e + 1], sl2s, -lse2k));
-          if constexpr (kDK) pk[e >> 1] = pack_bf16(p0 * fmaf(dp_[e], dpm, dsm), p1 * fmaf(dp_[e + 1], dpm, dsm));
-          else pk[e >> 1] = pack_bf16(p0, p1);
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 16; e += 2) {
-          const int i0 = 8 * (e >> 2) + 4 * half + (e & 3), i1 = i0 + 1;
-          const bool ok0 = kok && i0 >= ilo_r, ok1 = kok && i1 >= ilo_r;
-          const float p0 = ok0 ? fast_exp2(fmaf(s_[e], sl2s, -lse2)) : 0.f;
-          const float p1 = ok1 ? fast_exp2(fmaf(s_[e + 1], sl2s, -lse2)) : 0.f;
-          if constexpr (kDK) pk[e >> 1] = pack_bf16(p0 * fmaf(dp_[e], dpm, dsm), p1 * fmaf(dp_[e + 1], dpm, dsm));
-          else pk[e >> 1] = pack_bf16(p0, p1);
-        }
-      }
-      const bf16x8 b0 = __builtin_bit_cast(bf16x8, u32x4{pk[0], pk[1], pk[2], pk[3]});
-      const bf16x8 b1 = __builtin_bit_cast(bf16x8, u32x4{pk[4], pk[5], pk[6], pk[7]});
-      if constexpr (kDK) OPK::template tr_acc<RSA, kPF>(acc, At_r, 0, lane, b0, b1);
-      else OPV::template tr_acc<RSB, kPF>(acc, Bt_r, 0, lane, b0, b1);
-    };
-    accumulate(sv, dp, ilo, At, Bt);
-#pragma unroll
-    for (int r = 1; r < NR; ++r) {
-      const int ilo_r = ilo + 32 * r;  // first valid row of group r (rows j = t - 32r - 31 + i)
-      if (ilo_r >= 32) break;          // group r lies before the short window (uniform)
-      const char* Ar = At + r * TAB;
-      const floatx16 sr = OPK::template rows_x<RSA, kPF>(Ar, 0, lane, kf);
-      floatx16 dr;
-      if constexpr (kDK) dr = OPV::template rows_x<RSB, kPF>(Ar + TA, 0, lane, vf);
-      accumulate(sr, dr, ilo_r, Ar, Ar + TA);
-    }
-  }
-
-  write_out();
-}
-
-// dk2 or dv2 (mode 1 / 2) = the sum of the walk splits' fp32 sums in split
-// order; 4 values per thread
-template <int XW>
-__global__ __launch_bounds__(256) void bwd_dkv2_sum_kernel(BwdParams p, int splits, int mode) {
-  const int64_t i = (int64_t)bid_x() * 256 + tid_x();
-  const int64_t rows = (int64_t)p.tokens * p.hk;
-  if (i >= rows * (XW / 4)) return;
-  const int64_t row = i / (XW / 4);
-  const int c = (int)(i % (XW / 4)) * 4;
-  const float* src = p.dkv2s + row * XW + c;
-  floatx4 acc = *(const floatx4*)src;
-  for (int k = 1; k < splits; ++k) {
-    const floatx4 x = *(const floatx4*)(src + (int64_t)k * rows * XW);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] += x[e];
-  }
-  const int64_t t = row / p.hk, g = row % p.hk;
-  bf16* o = mode == 1 ? (bf16*)p.dk2 + t * p.dk_st + g * p.dk_sh : (bf16*)p.dv2 + t * p.dv_st + g * p.dv_sh;
-  bf16x4 b;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) b[e] = (bf16)acc[e];
-  *(bf16x4*)(o + c) = b;
-}
-
-// LDS bytes of a dk2 / dv2 workgroup (EW: bf16 units per row element)
-constexpr size_t dkv2_lds_bytes(int dk, int dv, int nr, int nwk, int ew) {
-  const size_t rsa = 2 * ew * dk + 32, rsb = 2 * ew * dv + 32, rkv = 2 * ew * (dk + dv);
-  const size_t ss = (2 * rkv + 1023) / 1024 * 1024;  // stage slot
-  return 2 * nr * 32 * (rsa + rsb) + 64 * nr * rkv + 3 * ss + (size_t)nwk * 64 * 16;
-}
-
-template <int DK, int DV, int NR, bool PH, bool F32, int NWK>
-hipError_t launch_dkv2_t(const BwdParams& p, int splits, hipStream_t stream) {
-  constexpr size_t lds = dkv2_lds_bytes(DK, DV, NR, NWK, F32 ? 2 : 1);
-  // more short-key rows than one launch's LDS holds: two launches (phases 1, 2)
-  const bool two = PH && p.ws > 32 * NR;
-  if (two || F32 || !p.dkv2s) splits = 1;
-  const int nblocks = (p.tokens + 32 * NWK - 1) / (32 * NWK) * p.hk * splits;
-  // fp32: one launch for both gradients (mode 3); bf16: dK2, then dV2
-  for (int mode = F32 ? 3 : 1; mode <= (F32 ? 3 : 2); ++mode) {
-    auto kern = [&]() {
-      if constexpr (F32) return bwd_dkv2_mfma_kernel<DK, DV, 3, NWK, NR, PH, true>;
-      else return mode == 1 ? bwd_dkv2_mfma_kernel<DK, DV, 1, NWK, NR, PH, false>
-                            : bwd_dkv2_mfma_kernel<DK, DV, 2, NWK, NR, PH, false>;
-    }();
-    hipError_t e = set_lds_limit((const void*)kern, lds);
-    if (e != hipSuccess) return e;
-    for (int phase = two ? 1 : 0; phase <= (two ? 2 : 0); ++phase) {
-      hipLaunchKernelGGL(kern, dim3(nblocks), dim3(64 * NWK), lds, stream, p, nblocks, phase, splits);
-      e = hipGetLastError();
-      if (e != hipSuccess) return e;
-    }
-    if (splits > 1) {
-      const int xw = mode == 1 ? DK : DV;
-      const dim3 grid((unsigned)(((int64_t)p.tokens * p.hk * (xw / 4) + 255) / 256));
-      if (xw == 64) hipLaunchKernelGGL(bwd_dkv2_sum_kernel<64>, grid, dim3(256), 0, stream, p, splits, mode);
-      else hipLaunchKernelGGL(bwd_dkv2_sum_kernel<128>, grid, dim3(256), 0, stream, p, splits, mode);
-      e = hipGetLastError();
-      if (e != hipSuccess) return e;
-    }
-  }
-  return hipSuccess;
-}
-
-template <int DK, int DV, int NR, bool PH, bool F32 = false>
-hipError_t launch_dkv2_w(const BwdParams& p, hipStream_t stream) {
-  const Dkv2Plan pl = bwd_dkv2_plan(p.tokens, p.hk, DK, DV, p.ws, p.wl, F32, device_cu_count());
-  if constexpr (DK == 128 && DV == 128 && !F32) {
-    if (pl.nwk == 8) return launch_dkv2_t<DK, DV, NR, PH, F32, 8>(p, pl.splits, stream);
-  }
-  return launch_dkv2_t<DK, DV, NR, PH, F32, 4>(p, pl.splits, stream);
-}
-
-template <int DK, int DV>
-hipError_t launch_dkv2_d(const BwdParams& p, hipStream_t stream) {
-  if constexpr (DK > 128) {
-    return launch_dkv2_w<DK, DV, 1, true>(p, stream);  // LDS for one row group per launch
-  } else {
-    if (p.ws <= 32) return launch_dkv2_w<DK, DV, 1, false>(p, stream);
-    if (p.ws <= 64) return launch_dkv2_w<DK, DV, 2, false>(p, stream);
-    return launch_dkv2_w<DK, DV, 2, true>(p, stream);  // two launches of two row groups
-  }
-}
-
-// bf16, score width DK and value width DV each 64 or 128, or DK = 256 over
-// DV = 128 or 256 (the dq and dk1 / dv1 passes only), 16-byte aligned rows;
-// fp32 inputs (p.f32, with the hi/lo rows of k2 and v2): DK == DV in {64, 128}.
-bool bwd_mfma_ok(const BwdParams& p) {
-  if (!p.mfma) return false;
-  if (p.f32 && (p.d != p.dv || (p.d != 64 && p.d != 128) || !p.k2s || !p.v2s)) return false;
-  const bool narrow = (p.d == 64 || p.d == 128) && (p.dv == 64 || p.dv == 128);
-  if (!narrow && !(p.d == 256 && (p.dv == 128 || p.dv == 256))) return false;
-  const int64_t st[] = {p.q_st, p.q_sh, p.k_st, p.k_sh, p.v_st, p.v_sh, p.do_st, p.do_sh};
-  for (int64_t s : st)
-    if (s % 8) return false;
-  const uintptr_t ptrs = (uintptr_t)p.q | (uintptr_t)p.k1 | (uintptr_t)p.k2 | (uintptr_t)p.v1 |
-                         (uintptr_t)p.v2 | (uintptr_t)p.dout;
-  // gradients are written 4 elements at a time
-  const int64_t ost[] = {p.dq_st, p.dq_sh, p.dk_st, p.dk_sh, p.dv_st, p.dv_sh};
-  for (int64_t s : ost)
-    if (s % 4) return false;
-  const uintptr_t optrs = (uintptr_t)p.dq | (uintptr_t)p.dk1 | (uintptr_t)p.dk2 | (uintptr_t)p.dv1 | (uintptr_t)p.dv2;
-  return (ptrs & 15) == 0 && (optrs & 15) == 0;
-}
-
 // fn(DK, DV) with the widths as integral constants; WIDE: DK = 256 as well
 template <bool WIDE, typename Fn>
 hipError_t by_widths(const BwdParams& p, Fn&& fn) {
@@ -1897,31 +1210,25 @@ BwdGeo base_geo(const BwdParams& p) {
 
 }  // namespace
 
-// Keys per workgroup (32 per wave, NWK waves): 8 waves when both widths are
-// 128 (bf16), 4 otherwise (at DK = 256 and for fp32 the 4 waves fill a CU's
-// LDS or registers).  When 8-wave workgroups would leave CUs without work --
-// few KV heads over few tokens, e.g. the reference adapter's 2 KV heads x
-// 16K tokens: 128 workgroups of 256 keys for 256 CUs -- 4-wave ones run, and
-// at bf16 widths <= 128 with one launch (short window <= 64) each (key block,
-// KV head) walk is cut into as many pieces as fill the CUs' resident
-// workgroup slots (two waves per SIMD, or what the LDS allows), up to 8 and
-// at least 128 queries per piece: the pieces' fp32 sums are added in a fixed
-// order.  Narrower workgroups alone measured slower (every workgroup forms
-// all 32 A / B rows of each step, so that work grows with the workgroup
-// count); a split walk forms each step's rows once, as before.
-Dkv2Plan bwd_dkv2_plan(int tokens, int hk, int d, int dv, int ws, int wl, bool f32, int cus) {
-  const int nr = ws <= 32 ? 1 : 2;  // row groups per launch at widths <= 128
-  const int64_t blocks8 = (int64_t)(tokens + 255) / 256 * hk;
-  if (!f32 && d == 128 && dv == 128 && blocks8 >= (nr == 1 ? 2 : 1) * (int64_t)cus) return {8, 1};
-  constexpr int nwk = 4;
-  if (f32 || d > 128 || dv > 128 || ws > 64 || tokens <= 0 || hk <= 0) return {nwk, 1};
-  const int64_t blocks = (int64_t)(tokens + 32 * nwk - 1) / (32 * nwk) * hk;
-  const int64_t by_lds = (int64_t)kLdsPerCu / dkv2_lds_bytes(d, dv, nr, nwk, 1);
-  const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(by_lds, 8 / nwk));
-  int64_t splits = ((int64_t)cus * per_cu + blocks - 1) / blocks;
-  splits = std::min<int64_t>(splits, kMaxWalkSplits);
-  splits = std::min<int64_t>(splits, ((int64_t)32 * nwk + wl - 1) / 128);  // pieces of >= 128 queries
-  return {nwk, (int)std::max<int64_t>(splits, 1)};
+// bf16, score width DK and value width DV each 64 or 128, or DK = 256 over
+// DV = 128 or 256 (the dq and dk1 / dv1 passes only), 16-byte aligned rows;
+// fp32 inputs (p.f32, with the hi/lo rows of k2 and v2): DK == DV in {64, 128}.
+bool bwd_mfma_ok(const BwdParams& p) {
+  if (!p.mfma) return false;
+  if (p.f32 && (p.d != p.dv || (p.d != 64 && p.d != 128) || !p.k2s || !p.v2s)) return false;
+  const bool narrow = (p.d == 64 || p.d == 128) && (p.dv == 64 || p.dv == 128);
+  if (!narrow && !(p.d == 256 && (p.dv == 128 || p.dv == 256))) return false;
+  const int64_t st[] = {p.q_st, p.q_sh, p.k_st, p.k_sh, p.v_st, p.v_sh, p.do_st, p.do_sh};
+  for (int64_t s : st)
+    if (s % 8) return false;
+  const uintptr_t ptrs = (uintptr_t)p.q | (uintptr_t)p.k1 | (uintptr_t)p.k2 | (uintptr_t)p.v1 |
+                         (uintptr_t)p.v2 | (uintptr_t)p.dout;
+  // gradients are written 4 elements at a time
+  const int64_t ost[] = {p.dq_st, p.dq_sh, p.dk_st, p.dk_sh, p.dv_st, p.dv_sh};
+  for (int64_t s : ost)
+    if (s % 4) return false;
+  const uintptr_t optrs = (uintptr_t)p.dq | (uintptr_t)p.dk1 | (uintptr_t)p.dk2 | (uintptr_t)p.dv1 | (uintptr_t)p.dv2;
+  return (ptrs & 15) == 0 && (optrs & 15) == 0;
 }
 
 hipError_t launch_bwd_dq_mfma(const BwdParams& p, hipStream_t stream) {
@@ -1968,17 +1275,6 @@ hipError_t launch_bwd_dv1_sum(const BwdParams& p, hipStream_t stream) {
   q.dk_sh = p.dv_sh;
   q.d = p.dv;
   return launch_bwd_dk1_sum(q, stream);
-}
-
-hipError_t launch_bwd_dkv2_mfma(const BwdParams& p, hipStream_t stream) {
-  if (p.f32) {  // fp32: one 32-row group of short keys
-    if (!bwd_mfma_ok(p) || p.ws > 32) return hipErrorNotSupported;
-    return p.d == 64 ? launch_dkv2_w<64, 64, 1, false, true>(p, stream) : launch_dkv2_w<128, 128, 1, false, true>(p, stream);
-  }
-  // one launch covers 64 short keys (32 at DK = 256); two launches over the fp32 partial twice that
-  const int one = p.d > 128 ? 32 : 64;
-  if (!bwd_mfma_ok(p) || p.ws > 2 * one || (p.ws > one && !p.dkv2p)) return hipErrorNotSupported;
-  return by_widths<true>(p, [&](auto dk, auto dv) { return launch_dkv2_d<decltype(dk)::value, decltype(dv)::value>(p, stream); });
 }
 
 }  // namespace sa

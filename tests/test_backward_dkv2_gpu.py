@@ -1,0 +1,44 @@
+"""dk2 / dv2 pass at the edges of its steps and walks: short windows at and
+around the 8- and 16-key steps (two or four units per 32-row step), groups that
+leave the last step partly filled, key blocks of 256 and 128 with a remainder,
+row groups past the first, and sequences that end inside a key block.  Checked
+with all five gradients against the portable kernels (same rounding points,
+another order of the fp32 sums: 2e-2 of the largest gradient in bf16, 1e-4 in
+fp32) and for repeatability."""
+
+import pytest
+import torch
+
+from helpers import rand_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,hq,hk,d,ws,wl,dtype", [
+    (300, 2, 2, 128, 16, 40, "bf16"),    # two units per step, one head: query pairs
+    (259, 3, 1, 128, 9, 300, "bf16"),    # ... three heads: steps straddle queries, odd unit count
+    (131, 6, 3, 64, 8, 20, "bf16"),      # four units: pairs of heads of two queries
+    (97, 8, 2, 128, 1, 1, "bf16"),       # one pair per query
+    (70, 5, 1, 64, 7, 33, "bf16"),       # 8 keys or fewer, odd group: two units
+    (513, 1, 1, 128, 17, 64, "bf16"),    # one unit per step again, a key past two blocks
+    (140, 4, 2, 256, 16, 50, "bf16"),    # width 256
+    (200, 4, 1, 256, 64, 100, "bf16"),   # ... two row groups in one walk
+    (150, 2, 1, 64, 128, 140, "bf16"),   # four row groups
+    (257, 6, 2, 128, 8, 30, "f32"),
+    (129, 3, 3, 64, 16, 129, "f32"),
+])
+def test_dkv2_step_edges(cuda, n, hq, hk, d, ws, wl, dtype):
+    from archlab_amd import simplicial_varlen_attention
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    x = [t[0].to(cuda) for t in rand_inputs(1, n, hq, hk, d, seed=n + ws, dtype=dt)]
+    cu = torch.tensor([0, 1, n // 3, n // 3 + 5, n], dtype=torch.int32, device=cuda)
+    dout = torch.randn(n, hq, d, generator=torch.Generator().manual_seed(n)).to(dt).to(cuda)
+    runs = []
+    for kernel in ("auto", "auto", "generic"):
+        xd = [t.clone().requires_grad_(True) for t in x]
+        simplicial_varlen_attention(*xd, cu, ws, wl, kernel=kernel).backward(dout)
+        runs.append([t.grad.float() for t in xd])
+    tol = 2e-2 if dtype == "bf16" else 1e-4
+    for name, a, a2, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), *runs):
+        assert torch.isfinite(a).all() and torch.equal(a, a2), name
+        assert (a - b).abs().max().item() <= tol * max(b.abs().max().item(), 1.0), name
