@@ -91,7 +91,14 @@ enum {
    * partials (those take 16-17.5x the bytes of q per 32 keys of short
    * window); the backward runs one more recomputation pass (about 20 % more
    * time at the benchmark shape). */
-  SA_FLAG_SEPARATE_DK1 = 2
+  SA_FLAG_SEPARATE_DK1 = 2,
+  /* Paged calls whose windows are consecutive blocks (contiguous decodes):
+   * token i is sequence i at position long_window - 1.  Position p of sequence
+   * s is block s * lt_stride + p of the long cache, and position p >=
+   * long_window - short_window is block s * st_stride + p - (long_window -
+   * short_window) of the short one.  Both tables and both token arrays are
+   * NULL, block_size is 1, both table widths are at least long_window. */
+  SA_FLAG_CONSECUTIVE_ROWS = 4
 };
 
 typedef struct sa_prefill_args {
@@ -236,7 +243,10 @@ int sa_paged_splits(const sa_paged_args* args);
 
 /* Name of the kernel family a call with these arguments runs: "mfma" (bf16
  * matrix-core path) or "generic" (portable path, fp32 and other shapes);
- * NULL if the arguments are invalid. */
+ * NULL if the arguments are invalid.  (Paged "generic" includes the fp32
+ * matrix kernel of fp32 queries over caches that are not both bf16; it merges
+ * split partials in sa_paged_workspace_bytes() of workspace, and does without
+ * splits where the caller brings none.) */
 const char* sa_prefill_kernel(const sa_prefill_args* args);
 const char* sa_paged_kernel(const sa_paged_args* args);
 

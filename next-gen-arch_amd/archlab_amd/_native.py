@@ -21,6 +21,7 @@ SA_DTYPE_F32, SA_DTYPE_BF16, SA_DTYPE_F16 = 0, 1, 2
 SA_INDEX_I32, SA_INDEX_I64 = 0, 1
 SA_FLAG_FORCE_GENERIC = 1
 SA_FLAG_SEPARATE_DK1 = 2
+SA_FLAG_CONSECUTIVE_ROWS = 4
 # SIMPLICIAL_MI355X_ABI_VERSION of the header these struct layouts mirror
 ABI_VERSION = 3
 

@@ -116,23 +116,52 @@ def _paged_launch(q, short_cache, long_cache, block_table, long_block_table, tok
         out = torch.empty((0, heads, dim), device=q.device, dtype=torch.float32)
         return (out, torch.empty((0, heads), device=q.device, dtype=torch.float32)) if return_lse else out
     token_seq, token_pos = token_seq.contiguous(), token_pos.contiguous()
-    lib = _native.load()
     out = torch.empty((tokens, heads, dim), device=q.device, dtype=torch.float32)
     lse = torch.empty((tokens, heads), device=q.device, dtype=torch.float32) if return_lse else None
     if window_caps is not None:
         window_caps = window_caps.to(torch.int32).contiguous()
     args = _paged_args(q, short_cache, long_cache, block_table, long_block_table, token_seq, token_pos,
                        short_window, long_window, scale, splits, out, lse, flags, window_caps=window_caps)
+    _run_paged(args, q.device, kernel)
+    return (out, lse) if return_lse else out
+
+
+def _rows_launch(q, short_cache, long_cache, short_window, long_window, scale, kernel):
+    """The launch behind ``window_decode``: token i attends to the first
+    ``short_window`` and ``long_window`` rows of batch element i of caches with
+    a block size of one row (``shape``, ``stride()``, ``rows_per_batch``), no
+    tables."""
+    tokens, heads, dim = q.shape
+    out = torch.empty((tokens, heads, dim), device=q.device, dtype=torch.float32)
+    if tokens == 0:
+        return out
+    args = _native.PagedArgs(
+        q=q.data_ptr(), q_stride_t=q.stride(0), q_stride_h=q.stride(1),
+        short_cache=short_cache.data_ptr(), sc_stride=(ctypes.c_int64 * 4)(*short_cache.stride()[:4]),
+        long_cache=long_cache.data_ptr(), lc_stride=(ctypes.c_int64 * 4)(*long_cache.stride()[:4]),
+        st_stride=short_cache.rows_per_batch, lt_stride=long_cache.rows_per_batch,
+        out=out.data_ptr(), o_stride_t=out.stride(0), o_stride_h=out.stride(1),
+        tokens=tokens, heads_q=heads, heads_kv=short_cache.shape[3], head_dim=dim, block_size=1,
+        num_seqs=tokens, short_table_width=long_window, long_table_width=long_window,
+        short_blocks=short_cache.shape[1], long_blocks=long_cache.shape[1],
+        short_window=short_window, long_window=long_window, scale=float(scale),
+        q_dtype=_native.dtype_code(q.dtype), cache_dtype=_native.cache_dtype_code(short_cache.dtype),
+        long_cache_dtype=_native.cache_dtype_code(long_cache.dtype),
+        flags=_kernel_flag(kernel) | _native.SA_FLAG_CONSECUTIVE_ROWS)
+    _run_paged(args, q.device, kernel)
+    return out
+
+
+def _run_paged(args, device, kernel):
+    lib = _native.load()
     if kernel == "mfma" and lib.sa_paged_kernel(ctypes.byref(args)) != b"mfma":
         raise ValueError("the MFMA kernel does not cover this dtype / head_dim / layout")
     nbytes = lib.sa_paged_workspace_bytes(ctypes.byref(args))
-    workspace = torch.empty(max(nbytes, 1) + 256, device=q.device, dtype=torch.uint8)
+    workspace = torch.empty(max(nbytes, 1) + 256, device=device, dtype=torch.uint8)
     base = workspace.data_ptr()
     aligned = (base + 255) & ~255
-    with torch.cuda.device(q.device):
-        _native.check(lib.sa_paged_fwd(ctypes.byref(args), aligned, nbytes,
-                                       _native.stream_handle(q.device)))
-    return (out, lse) if return_lse else out
+    with torch.cuda.device(device):
+        _native.check(lib.sa_paged_fwd(ctypes.byref(args), aligned, nbytes, _native.stream_handle(device)))
 
 
 def paged_plan(q, short_cache, long_cache, block_table, token_seq, token_pos, *, short_window,

@@ -6,8 +6,10 @@ short-axis rows (k1, v1) [B, N1, HK, D] and the long-axis rows (k2, v2)
 [B, N2, HK, D] that the single query attends to: every (j, k) pair of those
 rows is valid.  This module expresses that as a paged call: the rows become
 caches with a block size of one row, the query sits at position P, the long
-rows occupy positions P-L+1 .. P and the short rows P-N1+1 .. P, and the two
-block tables map each position to its row.  Nothing is copied: K and V stay
+rows occupy positions P-L+1 .. P and the short rows P-N1+1 .. P.  Where the
+lengths are known on the host the rows are consecutive blocks of the caches and
+the call carries no tables (SA_FLAG_CONSECUTIVE_ROWS); the bounded form maps
+each position to its row in two block tables.  Nothing is copied: K and V stay
 separate tensors and the cache's K-to-V stride is the distance between them.
 """
 
@@ -15,7 +17,7 @@ from __future__ import annotations
 
 import torch
 
-from .simplicial_paged import _paged_launch
+from .simplicial_paged import _paged_launch, _rows_launch
 
 
 class _KVPair:
@@ -24,7 +26,8 @@ class _KVPair:
     stride is the element distance from K's first element to V's (it may be
     negative), a block is one row."""
 
-    def __init__(self, k, v):
+    def __init__(self, k, v, first=0):
+        # ``first``: rows before it are left out of every batch element
         b, n, hk, d = k.shape
         es = k.element_size()
 
@@ -38,12 +41,13 @@ class _KVPair:
         # of a longer cache keeps its own row stride, no copy)
         self.rows_per_batch = k.stride(0) // k.stride(1) if b > 1 else n
         self._k, self._v = k, v  # keep both alive for the launch
-        self.shape = (2, b * self.rows_per_batch, 1, hk, d)
+        self.shape = (2, b * self.rows_per_batch - first, 1, hk, d)
+        self._offset = first * k.stride(1) * es
         self.dtype = k.dtype
         self._strides = ((v.data_ptr() - k.data_ptr()) // es, k.stride(1), k.stride(1), k.stride(2), 1)
 
     def data_ptr(self):
-        return self._k.data_ptr()
+        return self._k.data_ptr() + self._offset
 
     def stride(self, dim=None):
         return self._strides if dim is None else self._strides[dim]
@@ -60,21 +64,9 @@ def window_decode(q, k1, k2, v1, v2, scale, key_lower=0, kernel="auto"):
     length = n2 - key_lower
     if not 1 <= n1 <= length:
         raise ValueError("the short axis must not be longer than the long axis")
-    dev = q.device
-    long_cache = _KVPair(k2, v2)
-    short_cache = _KVPair(k1, v1)
-    pos = length - 1  # query position; long rows key_lower.. sit at positions 0..length-1
-    p = torch.arange(length, device=dev, dtype=torch.int64)
-    rows = torch.arange(b, device=dev, dtype=torch.int64)[:, None]
-    long_table = (rows * long_cache.rows_per_batch + key_lower + p[None, :]).to(torch.int32)
-    short_row = (p - (length - n1)).clamp_min(0)  # positions before the short window map to row 0 (unused)
-    short_table = (rows * short_cache.rows_per_batch + short_row[None, :]).to(torch.int32)
-    token_seq = torch.arange(b, device=dev, dtype=torch.int32)
-    token_pos = torch.full((b,), pos, device=dev, dtype=torch.int32)
     if q.stride(-1) != 1:
         q = q.contiguous()
-    return _paged_launch(q, short_cache, long_cache, short_table, long_table, token_seq, token_pos,
-                         n1, length, scale, None, False, kernel)
+    return _rows_launch(q, _KVPair(k1, v1), _KVPair(k2, v2, first=key_lower), n1, length, scale, kernel)
 
 
 def window_decode_bounded(q, k1, k2, v1, v2, scale, lengths, max_short, kernel="auto"):

@@ -161,9 +161,16 @@ static int check_paged(const sa_paged_args* a) {
   if (a->tokens > 0 && (a->num_seqs < 1 || a->short_table_width < 1 || a->long_table_width < 1 ||
                         a->short_blocks < 1 || a->long_blocks < 1))
     return fail(SA_ERR_INVALID, "invalid paged simplicial inputs");
-  if (a->tokens > 0 && (!a->q || !a->short_cache || !a->long_cache || !a->short_table || !a->long_table ||
-                        !a->token_seq || !a->token_pos || !a->out))
+  // SA_FLAG_CONSECUTIVE_ROWS: the tables and the token arrays are implied
+  const bool implied = a->flags & SA_FLAG_CONSECUTIVE_ROWS;
+  if (a->tokens > 0 && (!a->q || !a->short_cache || !a->long_cache || !a->out ||
+                        (!implied && (!a->short_table || !a->long_table || !a->token_seq || !a->token_pos))))
     return fail(SA_ERR_INVALID, "null tensor pointer");
+  if (implied && (a->short_table || a->long_table || a->token_seq || a->token_pos || a->num_seqs < a->tokens))
+    return fail(SA_ERR_INVALID, "consecutive rows take no tables or token arrays");
+  if (implied && (a->block_size != 1 || a->short_table_width < a->long_window ||
+                  a->long_table_width < a->long_window))
+    return fail(SA_ERR_INVALID, "consecutive rows: block_size 1, table widths of at least long_window");
   return SA_OK;
 }
 
@@ -276,7 +283,8 @@ int sa_paged_fwd(const sa_paged_args* a, void* workspace, size_t workspace_bytes
   int rc = sa::check_paged(a);
   if (rc != SA_OK) return rc;
   if (a->tokens == 0) return SA_OK;
-  const sa_paged_args c = sa::clip_paged(a);
+  sa_paged_args c = sa::clip_paged(a);
+  if (workspace_bytes == 0 && sa::paged_f32_route(&c)) sa::paged_without_partials(&c);
   const int splits = sa::paged_choose_splits(&c);
   const size_t need = sa::paged_workspace_bytes(&c, splits);
   if (workspace_bytes < need) return sa::fail(SA_ERR_INVALID, "workspace too small");
@@ -292,7 +300,8 @@ int sa_paged_fwd_noalloc(const sa_paged_args* a, sa_stream_t stream) {
   int rc = sa::check_paged(a);
   if (rc != SA_OK) return rc;
   if (a->tokens == 0) return SA_OK;
-  const sa_paged_args c = sa::clip_paged(a);
+  sa_paged_args c = sa::clip_paged(a);
+  if (sa::paged_f32_route(&c)) sa::paged_without_partials(&c);
   const int splits = sa::paged_choose_splits(&c);
   const size_t need = sa::paged_workspace_bytes(&c, splits);
   if (need > sa::kScratchBytes)

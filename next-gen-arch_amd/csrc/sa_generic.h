@@ -59,6 +59,7 @@ __device__ __forceinline__ int64_t clamp64(int64_t x, int64_t lo, int64_t hi) { 
 __device__ __forceinline__ int64_t block_of(const void* table, int is64, int64_t row_stride, int width, int64_t nblocks,
                                             int64_t seq, int pos, int block_size) {
   const int64_t col = clamp64(pos / block_size, 0, width - 1);
+  if (table == nullptr) return clamp64(seq * row_stride + col, 0, nblocks - 1);  // consecutive blocks
   return clamp64(load_index(table, seq * row_stride + col, is64), 0, nblocks - 1);
 }
 
@@ -78,7 +79,9 @@ struct PagedRows {
   int st_w, lt_w;
   int64_t s_blocks, l_blocks;
   int64_t seq;
+  int s_shift;  // positions before the first short row (consecutive rows; 0 with tables)
   __device__ int64_t s_off(int pos, int g) const {
+    if (s_shift) pos = max(pos - s_shift, 0);
     const int64_t blk = block_of(stable, stab64, st_s, st_w, s_blocks, seq, pos, block_size);
     return blk * sc_b + (int64_t)(pos % block_size) * sc_s + (int64_t)g * sc_h;
   }

@@ -38,6 +38,21 @@ int paged_choose_splits(const sa_paged_args* a);
 size_t paged_workspace_bytes(const sa_paged_args* a, int splits);
 hipError_t launch_paged(const sa_paged_args* a, int splits, void* ws, size_t ws_bytes, hipStream_t stream);
 
+struct PagedRows;  // sa_generic.h
+PagedRows paged_rows(const sa_paged_args* a);
+// Merge of P partials per (token, head) into a->out / a->lse, in partial order.
+hipError_t launch_paged_combine(const float* part_o, const float* part_m, const float* part_z, int P,
+                                const sa_paged_args* a, hipStream_t stream);
+
+// fp32 query over caches that are not both bf16 (sa_paged_f32.hip).
+bool paged_f32_route(const sa_paged_args* a);
+// Fixes the form that needs no workspace, for callers that bring none: one
+// split, or the portable kernel where rows of a head merge through partials.
+void paged_without_partials(sa_paged_args* a);
+int paged_f32_splits(const sa_paged_args* a);
+size_t paged_f32_workspace_bytes(const sa_paged_args* a, int splits);
+hipError_t launch_paged_f32(const sa_paged_args* a, int splits, void* ws, size_t ws_bytes, hipStream_t stream);
+
 // Backward (sa_backward.hip).
 size_t prefill_bwd_workspace_bytes(const sa_prefill_bwd_args* a);
 hipError_t launch_prefill_bwd(const sa_prefill_bwd_args* a, void* ws, hipStream_t stream);

@@ -36,6 +36,7 @@ struct PagedParams {
   int64_t st_s, lt_s;
   const void* tseq;
   const void* tpos;
+  int s_shift;  // positions before the first short row (consecutive rows)
   int stab64, ltab64, seq64, pos64;  // index widths (int64 when set)
   int st_w, lt_w, num_seqs;
   int64_t s_blocks, l_blocks;
@@ -91,9 +92,11 @@ __global__ __launch_bounds__(64 * NW, (D >= 256 || NW < 4 ? 1 : 2)) void paged_m
   const int token = b / p.hk;
 
   // per-token scalars, both index loads in one round trip (uniform: SGPRs)
-  const int seq_raw = (int)clamp64(p.seq64 ? ((const int64_t*)p.tseq)[token] : ((const int32_t*)p.tseq)[token], 0,
-                                   p.num_seqs - 1);
-  const int pos_raw = (int)(p.pos64 ? ((const int64_t*)p.tpos)[token] : ((const int32_t*)p.tpos)[token]);
+  const int seq_raw = !p.tseq ? token
+                              : (int)clamp64(p.seq64 ? ((const int64_t*)p.tseq)[token]
+                                                     : ((const int32_t*)p.tseq)[token], 0, p.num_seqs - 1);
+  const int pos_raw = !p.tpos ? p.wl - 1
+                              : (int)(p.pos64 ? ((const int64_t*)p.tpos)[token] : ((const int32_t*)p.tpos)[token]);
   // per-token window limits (the chunk grid stays the one of p.wl)
   int ws_t = p.ws, wl_t = p.wl;
   if (p.caps) {
@@ -162,11 +165,17 @@ __global__ __launch_bounds__(64 * NW, (D >= 256 || NW < 4 ? 1 : 2)) void paged_m
       }
     };
     if (with_short) {  // issued with the long-table loads (uniform branches)
-      const int col = min(max(j, 0) / p.bs, p.st_w - 1);
-      sraw = p.stab64 ? ((const int64_t*)p.stable)[seq * p.st_s + col]
+      const int col = min(max(j - p.s_shift, 0) / p.bs, p.st_w - 1);
+      sraw = !p.stable ? seq * p.st_s + col : p.stab64 ? ((const int64_t*)p.stable)[seq * p.st_s + col]
                       : (int64_t)((const int32_t*)p.stable)[seq * p.st_s + col];
     }
-    if (p.ltab64) lookup(int64_t{});
+    if (!p.ltable) {  // consecutive blocks (uniform)
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int ps = seg_lo + min(i0 + tid + u * 64 * NW, nseg - 1);
+        raw[u] = seq * p.lt_s + min(ps / p.bs, p.lt_w - 1);
+      }
+    } else if (p.ltab64) lookup(int64_t{});
     else lookup(int32_t{});
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
@@ -414,29 +423,53 @@ __global__ __launch_bounds__(64 * NW, (D >= 256 || NW < 4 ? 1 : 2)) void paged_m
 }
 
 // Merge P = splits * row-groups partials per (token, head) in a fixed order.
-// One wave per (token, head); D/64 output values per lane.
+// One wave per (token, head), or from 8 partials on four waves that take every
+// fourth one; D/64 output values per lane.  The maxima and sums of 64 partials
+// are read at once, one per lane, and the partial outputs are independent
+// loads: the merge waits for memory twice, not twice per partial.
+template <int NW>
 __global__ __launch_bounds__(256) void paged_combine_kernel(const float* __restrict__ part_o,
                                                             const float* __restrict__ part_m,
                                                             const float* __restrict__ part_z, int P, int tokens,
                                                             int hq, int D, float* __restrict__ out, int64_t o_st,
                                                             int64_t o_sh, float* __restrict__ lse) {
+  __shared__ float red[NW == 1 ? 1 : 4 * 256];
   const int wid = tid_x() >> 6, lane = tid_x() & 63;
-  const int64_t th = (int64_t)bid_x() * 4 + wid;
-  if (th >= (int64_t)tokens * hq) return;
+  const int64_t th = NW == 1 ? (int64_t)bid_x() * 4 + wid : bid_x();
+  if (th >= (int64_t)tokens * hq) return;  // (whole workgroups when NW == 4)
   const int token = (int)(th / hq), h = (int)(th % hq);
   const int64_t stride = (int64_t)tokens * hq;
   float M = -INFINITY;
-  for (int i = 0; i < P; ++i) M = fmaxf(M, part_m[i * stride + th]);
+  for (int i = lane; i < P; i += 64) M = fmaxf(M, part_m[i * stride + th]);
+  M = wave_max(M);
   float Z = 0.f;
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < P; ++i) {
-    const float mi = part_m[i * stride + th];
-    const float w = mi > -INFINITY ? fast_exp2(mi - M) : 0.f;
-    Z += w * part_z[i * stride + th];
-    const float* po = part_o + (i * stride + th) * D;
+  for (int i0 = 0; i0 < P; i0 += 64) {
+    const int n = min(64, P - i0);
+    float w = 0.f;  // weight of partial i0 + lane
+    if (lane < n) {
+      const float mi = part_m[(i0 + lane) * stride + th];
+      w = mi > -INFINITY ? fast_exp2(mi - M) : 0.f;
+      Z += w * part_z[(i0 + lane) * stride + th];
+    }
+    const float* po = part_o + ((int64_t)i0 * stride + th) * D + lane;
+#pragma unroll 4
+    for (int i = NW == 1 ? 0 : wid; i < n; i += NW) {
+      const float wi = __shfl(w, i);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (64 * s < D) acc[s] = fmaf(wi, po[(int64_t)i * stride * D + 64 * s], acc[s]);
+    }
+  }
+  Z = wave_sum(Z);
+  if (NW == 4) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) red[wid * 256 + 64 * s + lane] = acc[s];
+    __syncthreads();
+    if (wid) return;
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      if (64 * s < D) acc[s] += w * po[64 * s + lane];
+      acc[s] = (red[64 * s + lane] + red[256 + 64 * s + lane]) + (red[512 + 64 * s + lane] + red[768 + 64 * s + lane]);
   }
   const float inv = 1.f / Z;
   float* orow = out + (int64_t)token * o_st + (int64_t)h * o_sh;
@@ -444,6 +477,16 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(const float* __restr
   for (int s = 0; s < 4; ++s)
     if (64 * s < D) orow[64 * s + lane] = acc[s] * inv;
   if (lse && lane == 0) lse[th] = (M + __log2f(Z)) * kLn2;
+}
+
+hipError_t launch_paged_combine(const float* part_o, const float* part_m, const float* part_z, int P,
+                                const sa_paged_args* a, hipStream_t stream) {
+  const int64_t nth = (int64_t)a->tokens * a->heads_q;
+  const bool four = P >= 8;
+  hipLaunchKernelGGL(four ? paged_combine_kernel<4> : paged_combine_kernel<1>,
+                     dim3((unsigned)(four ? nth : (nth + 3) / 4)), dim3(256), 0, stream, part_o, part_m, part_z, P,
+                     a->tokens, a->heads_q, a->head_dim, a->out, a->o_stride_t, a->o_stride_h, a->lse);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -469,8 +512,8 @@ template <typename QT, typename SCT, typename LCT>
 __global__ __launch_bounds__(kGenThreads) void paged_generic_kernel(GenericPagedParams gp) {
   const int token = bid_x(), h = bid_y();
   PagedRows rows = gp.rows;
-  rows.seq = clamp64(load_index(gp.tseq, token, gp.seq64), 0, gp.num_seqs - 1);
-  const int pos = (int)load_index(gp.tpos, token, gp.pos64);
+  rows.seq = gp.tseq ? clamp64(load_index(gp.tseq, token, gp.seq64), 0, gp.num_seqs - 1) : token;
+  const int pos = gp.tpos ? (int)load_index(gp.tpos, token, gp.pos64) : gp.wl - 1;
   int ws = gp.ws, wl = gp.wl;
   if (gp.caps) {
     ws = max(1, min(ws, gp.caps[2 * token]));
@@ -484,6 +527,39 @@ __global__ __launch_bounds__(kGenThreads) void paged_generic_kernel(GenericPaged
 
 // ---------------------------------------------------------------------------
 // Host side
+
+// Consecutive rows: the short rows are the last short_window positions.
+static int rows_shift(const sa_paged_args* a) {
+  return a->flags & SA_FLAG_CONSECUTIVE_ROWS ? a->long_window - a->short_window : 0;
+}
+
+PagedRows paged_rows(const sa_paged_args* a) {
+  PagedRows rows{};
+  rows.sc = a->short_cache;
+  rows.lc = a->long_cache;
+  rows.sc_a = a->sc_stride[0];
+  rows.sc_b = a->sc_stride[1];
+  rows.sc_s = a->sc_stride[2];
+  rows.sc_h = a->sc_stride[3];
+  rows.lc_a = a->lc_stride[0];
+  rows.lc_b = a->lc_stride[1];
+  rows.lc_s = a->lc_stride[2];
+  rows.lc_h = a->lc_stride[3];
+  rows.stable = a->short_table;
+  rows.ltable = a->long_table;
+  rows.st_s = a->st_stride;
+  rows.lt_s = a->lt_stride;
+  rows.stab64 = a->table_index_dtype == SA_INDEX_I64;
+  rows.ltab64 = a->long_table_index_dtype == SA_INDEX_I64;
+  rows.st_w = a->short_table_width;
+  rows.lt_w = a->long_table_width;
+  rows.s_blocks = a->short_blocks;
+  rows.l_blocks = a->long_blocks;
+  rows.block_size = a->block_size;
+  rows.s_shift = rows_shift(a);
+  rows.seq = 0;
+  return rows;
+}
 
 int paged_mfma_supported(const sa_paged_args* a) {
   if (a->flags & SA_FLAG_FORCE_GENERIC) return 0;
@@ -511,7 +587,7 @@ static int paged_nw(const sa_paged_args* a) {
 // chunk count, and with it the split count and the workspace, stay bounded by
 // the block-table capacity whatever window a global layer passes.
 int paged_choose_splits(const sa_paged_args* a) {
-  if (!paged_mfma_supported(a)) return 1;
+  if (!paged_mfma_supported(a)) return paged_f32_route(a) ? paged_f32_splits(a) : 1;
   const int nc = (int)(((int64_t)a->long_window + kChunk - 1) / kChunk);
   if (a->splits > 0) return a->splits < nc ? a->splits : nc;
   const int group = a->heads_q / a->heads_kv;
@@ -534,7 +610,7 @@ int paged_choose_splits(const sa_paged_args* a) {
 }
 
 size_t paged_workspace_bytes(const sa_paged_args* a, int splits) {
-  if (!paged_mfma_supported(a)) return 0;
+  if (!paged_mfma_supported(a)) return paged_f32_route(a) ? paged_f32_workspace_bytes(a, splits) : 0;
   if (splits * ((a->short_window + 31) / 32) == 1) return 0;  // direct output, no partials
   const size_t P = (size_t)splits * ((a->short_window + 31) / 32);
   const size_t th = (size_t)a->tokens * a->heads_q;
@@ -630,6 +706,7 @@ hipError_t launch_paged(const sa_paged_args* a, int splits, void* ws, size_t ws_
     p.lt_s = a->lt_stride;
     p.tseq = a->token_seq;
     p.tpos = a->token_pos;
+    p.s_shift = rows_shift(a);
     p.stab64 = a->table_index_dtype == SA_INDEX_I64;
     p.ltab64 = a->long_table_index_dtype == SA_INDEX_I64;
     p.seq64 = a->token_index_dtype == SA_INDEX_I64;
@@ -684,38 +761,14 @@ hipError_t launch_paged(const sa_paged_args* a, int splits, void* ws, size_t ws_
     }
     if (e != hipSuccess) return e;
     if (p.direct) return hipSuccess;
-    const int64_t nth = (int64_t)a->tokens * a->heads_q;
-    hipLaunchKernelGGL(paged_combine_kernel, dim3((unsigned)((nth + 3) / 4)), dim3(256), 0, stream, p.part_o,
-                       p.part_m, p.part_z, (int)P, a->tokens, a->heads_q, a->head_dim, a->out, a->o_stride_t,
-                       a->o_stride_h, a->lse);
-    return hipGetLastError();
+    return launch_paged_combine(p.part_o, p.part_m, p.part_z, (int)P, a, stream);
   }
+  if (paged_f32_route(a)) return launch_paged_f32(a, splits, ws, ws_bytes, stream);
   GenericPagedParams gp{};
   gp.q = a->q;
   gp.q_st = a->q_stride_t;
   gp.q_sh = a->q_stride_h;
-  gp.rows.sc = a->short_cache;
-  gp.rows.lc = a->long_cache;
-  gp.rows.sc_a = a->sc_stride[0];
-  gp.rows.sc_b = a->sc_stride[1];
-  gp.rows.sc_s = a->sc_stride[2];
-  gp.rows.sc_h = a->sc_stride[3];
-  gp.rows.lc_a = a->lc_stride[0];
-  gp.rows.lc_b = a->lc_stride[1];
-  gp.rows.lc_s = a->lc_stride[2];
-  gp.rows.lc_h = a->lc_stride[3];
-  gp.rows.stable = a->short_table;
-  gp.rows.ltable = a->long_table;
-  gp.rows.st_s = a->st_stride;
-  gp.rows.lt_s = a->lt_stride;
-  gp.rows.stab64 = a->table_index_dtype == SA_INDEX_I64;
-  gp.rows.ltab64 = a->long_table_index_dtype == SA_INDEX_I64;
-  gp.rows.st_w = a->short_table_width;
-  gp.rows.lt_w = a->long_table_width;
-  gp.rows.s_blocks = a->short_blocks;
-  gp.rows.l_blocks = a->long_blocks;
-  gp.rows.block_size = a->block_size;
-  gp.rows.seq = 0;
+  gp.rows = paged_rows(a);
   gp.tseq = a->token_seq;
   gp.tpos = a->token_pos;
   gp.caps = a->token_window_caps;
