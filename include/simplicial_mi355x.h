@@ -208,6 +208,10 @@ typedef struct sa_prefill_bwd_args {
  *   value_dim]);
  * - for fp32 inputs on the matrix cores, k2 and v2 as hi/lo bf16 rows
  *   ([tokens][heads_kv][2 head_dim] each);
+ * - for bf16 at head_dim 512 over value_dim 256 and short windows <= 32, the
+ *   partials of dk1 and dv1 (24-25.5x the bytes of q at GQA groups of 4, up to
+ *   2 GiB; none with SA_FLAG_SEPARATE_DK1, which leaves those passes to the
+ *   portable kernels);
  * - for bf16 at widths 64 / 128 and short windows <= 64 whose (key block, KV
  *   head) work leaves CUs idle (few KV heads over few tokens), the fp32 sums of
  *   the dk2 / dv2 pass's walk pieces ([pieces <= 8][tokens][heads_kv]

@@ -61,6 +61,11 @@ inline int dq_queries_per_block(int group) { return group % 4 == 0 ? 1 : group %
 // portable pass runs instead.
 hipError_t launch_bwd_dq_mfma(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dkv1_mfma(const BwdParams& p, hipStream_t stream);
+// dq, dk1 and dv1 in one pass (sa_backward_dq.hip) with its partials in the
+// scratch_bytes at p.dkv2s, in place of the two passes above
+hipError_t launch_bwd_dq_core(const BwdParams& p, size_t scratch_bytes, hipStream_t stream);
+// its partials at score width 512
+size_t dq_core_partial_bytes(int tokens, int hq, int hk, int d, int dv, int ws);
 // scratch_bytes: the space at p.dkv2s
 hipError_t launch_bwd_dkv2_mfma(const BwdParams& p, size_t scratch_bytes, hipStream_t stream);
 // The dq pass can produce dk1 (p.dk1p set): the MFMA passes apply and the

@@ -623,11 +623,23 @@ static size_t dkv2_split_bytes(const sa_prefill_bwd_args* a) {
   if (splits <= 1) return 0;
   return ((size_t)splits * f.total_tokens * f.heads_kv * std::max(d, dv) * sizeof(float) + 255) & ~(size_t)255;
 }
+// Score width 512: the partials of the dq / dk1 / dv1 pass, up to kWidePartialCap
+// (past it the pass runs in phases; the dk2 / dv2 pieces reuse the space).
+constexpr size_t kWidePartialCap = (size_t)2 << 30;
+static size_t wide_partial_bytes(const sa_prefill_bwd_args* a) {
+  const sa_prefill_args& f = a->fwd;
+  if (f.dtype != SA_DTYPE_BF16 || (f.flags & (SA_FLAG_FORCE_GENERIC | SA_FLAG_SEPARATE_DK1)) || f.head_dim != 512 ||
+      f.value_dim != 256 || f.short_window > 32 || f.heads_kv <= 0)
+    return 0;
+  const size_t b = dq_core_partial_bytes(f.total_tokens, f.heads_q, f.heads_kv, f.head_dim, f.value_dim, f.short_window);
+  return std::min((b + 255) & ~(size_t)255, kWidePartialCap);
+}
 // The workspace: delta and dlse rows, the hi/lo rows of fp32 inputs, then the
 // scratch (dk1 and dv1 partials, reused by the dk2 / dv2 pieces).
 static size_t bwd_scratch_offset(const sa_prefill_bwd_args* a) { return 2 * bwd_row_bytes(a) + 2 * f32_split_bytes(a); }
 size_t prefill_bwd_workspace_bytes(const sa_prefill_bwd_args* a) {
-  return bwd_scratch_offset(a) + dk1_partial_bytes(a) + dv1_partial_bytes(a) + dkv2_long_bytes(a) + dkv2_split_bytes(a);
+  return bwd_scratch_offset(a) + dk1_partial_bytes(a) + dv1_partial_bytes(a) + dkv2_long_bytes(a) + dkv2_split_bytes(a) +
+         wide_partial_bytes(a);
 }
 
 template <typename T>
@@ -653,17 +665,20 @@ static hipError_t launch_bwd_t(const BwdParams& p, size_t scratch_bytes, hipStre
     if (e != hipSuccess) return e;
   }
   // each pass runs on MFMA tiles where its kernel covers the call, else on the portable kernel
-  e = launch_bwd_dq_mfma(p, stream);
+  e = launch_bwd_dq_core(p, scratch_bytes, stream);
+  const bool merged = e != hipErrorNotSupported;  // dq, dk1 and dv1 are done
+  if (!merged) e = launch_bwd_dq_mfma(p, stream);
   if (e == hipErrorNotSupported) {
     hipLaunchKernelGGL(bwd_dq_kernel<T>, ks[0].grid, dim3(kBwdThreads), ks[0].lds, stream, p);
     e = hipGetLastError();
   }
   if (e != hipSuccess) return e;
-  if (p.dk1p) {  // dk1 from the dq pass's partials; the dkv1 launch below computes dv1 only
+  if (p.dk1p && !merged) {  // dk1 from the dq pass's partials; the dkv1 launch below computes dv1 only
     e = launch_bwd_dk1_sum(p, stream);
     if (e != hipSuccess) return e;
   }
-  if (p.dv1p) {  // dv1 from the dq pass's partials as well: no dk1 / dv1 pass
+  if (merged) {
+  } else if (p.dv1p) {  // dv1 from the dq pass's partials as well: no dk1 / dv1 pass
     e = launch_bwd_dv1_sum(p, stream);
   } else {
     e = launch_bwd_dkv1_mfma(p, stream);

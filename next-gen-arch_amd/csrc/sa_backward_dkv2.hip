@@ -25,6 +25,10 @@
 // it now: one wave per SIMD issues at most one instruction every four cycles,
 // and a step's ~700 (64 of them MFMAs) take longer than its matrix work.
 //
+// Score width 512 (determinant form of 256-wide heads): the accumulators of
+// 512 + 256 columns do not fit; one launch takes dV2 and 128 columns of dK2, a
+// second one the other 384, with the scores formed in both.
+//
 // Walks are cut into pieces when the (key block, KV head) workgroups alone
 // leave CUs idle in the last wave of workgroups: each piece writes fp32 sums
 // that bwd_dkv2_sum_kernel adds in piece order (no atomics).
@@ -59,10 +63,10 @@ struct Dkv2Lds {
   static constexpr size_t bytes(int ring) { return 2 * TAB + (size_t)ring * RKV + 2 * PK * SS + NW * 64 * 16; }
 };
 
-template <int DK, int DV, int SETS, int PK, bool F32>
+template <int DK, int DV, int SETS, int PK, bool F32, int KB0, int KBN, int VBN>
 __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo geo) {
   using L = Dkv2Lds<DK, DV, PK, F32>;
-  using C = BwdCore<DK, DV, SETS, F32>;
+  using C = BwdCore<DK, DV, SETS, F32, KB0, KBN, VBN>;
   constexpr int NW = 4, KB = 128 * SETS, R = 32 / PK, EW = L::EW;
   constexpr int RBK = L::RBK, RKV = L::RKV, SS = L::SS, SI = L::SI, TAB = L::TAB;
   static_assert(!F32 || DK == DV, "fp32 inputs: equal widths");
@@ -121,23 +125,23 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
       if (geo.splits > 1) {
         float* part = p.dkv2s + (((int64_t)split * p.tokens + kw) * p.hk + g) * (DK + DV);
 #pragma unroll
-        for (int i = 0; i < (DK + DV) / 8; ++i) {
+        for (int i = 0; i < 4 * (KBN + VBN); ++i) {
           const int db = i >> 2, q4 = i & 3;
           floatx4 x;
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            x[e] = db < DK / 32 ? acc_get(core.ak[c][db < DK / 32 ? db : 0], 4 * q4 + e)
-                                : acc_get(core.av[c][db < DK / 32 ? 0 : db - DK / 32], 4 * q4 + e);
-          *(floatx4*)(part + 32 * db + 8 * q4 + 4 * hf) = x;
+            x[e] = db < KBN ? acc_get(core.ak[c][db < KBN ? db : 0], 4 * q4 + e)
+                            : acc_get(core.av[c][db < KBN ? 0 : db - KBN], 4 * q4 + e);
+          *(floatx4*)(part + (db < KBN ? 32 * (KB0 + db) : DK + 32 * (db - KBN)) + 8 * q4 + 4 * hf) = x;
         }
         continue;
       }
       const int64_t ok = (int64_t)kw * p.dk_st + (int64_t)g * p.dk_sh, ov = (int64_t)kw * p.dv_st + (int64_t)g * p.dv_sh;
 #pragma unroll
-      for (int db = 0; db < DK / 32; ++db) {
+      for (int db = 0; db < KBN; ++db) {
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) {
-          const int d = 32 * db + 8 * q4 + 4 * hf;
+          const int d = 32 * (KB0 + db) + 8 * q4 + 4 * hf;
           if constexpr (F32) {
             floatx4 x;
 #pragma unroll
@@ -152,7 +156,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
         }
       }
 #pragma unroll
-      for (int db = 0; db < DV / 32; ++db) {
+      for (int db = 0; db < VBN; ++db) {
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) {
           const int d = 32 * db + 8 * q4 + 4 * hf;
@@ -292,7 +296,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
   // (lane-derived values from a fresh lane id per step: held through the loop
   // they cost the registers of the fragments)
   struct Form {
-    u32x4 q, gr, a[UA], b[UB];
+    u32x4 q, gr, src[UA + UB];
     uint32_t lane;
   } fm;
   auto form_row = [&](uint32_t block, uint32_t segs) { return 8u * (uint32_t)wid + (block * 64u + fm.lane) / segs; };
@@ -315,10 +319,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
     fm.lane = (uint32_t)fresh_lane();
     fm.q = *(const u32x4*)(sr + 16 * (fm.lane % SK));
     fm.gr = *(const u32x4*)(sr + RBK + 16 * (fm.lane % SV));
-#pragma unroll
-    for (int u = 0; u < UA; ++u) fm.a[u] = *(const u32x4*)(form_src(st, x, form_row(u, SK)) + 16 * (fm.lane % SK));
-#pragma unroll
-    for (int u = 0; u < UB; ++u) fm.b[u] = *(const u32x4*)(form_src(st, x, form_row(u, SV)) + RBK + 16 * (fm.lane % SV));
+  };
+  auto form_read_block = [&](auto kk, int st, Unit x) {  // source rows of formed block k
+    constexpr int k = decltype(kk)::value;
+    if constexpr (k < UA) fm.src[k] = *(const u32x4*)(form_src(st, x, form_row(k, SK)) + 16 * (fm.lane % SK));
+    else fm.src[k] = *(const u32x4*)(form_src(st, x, form_row(k - UA, SV)) + RBK + 16 * (fm.lane % SV));
   };
   // block k of the formed rows (A blocks, then B blocks) into tile buffer buf
   auto form_block = [&](auto kk, int buf) {
@@ -328,7 +333,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
     char* const tile = lds + buf * TAB + (isa ? 0 : C::TK);
     const uint32_t row = form_row(isa ? k : k - UA, segs), sg = fm.lane % segs;
     const u32x4 x = isa ? fm.q : fm.gr;
-    const u32x4 y = isa ? fm.a[isa ? k : 0] : fm.b[isa ? 0 : k - UA];
+    const u32x4 y = fm.src[k];
     if constexpr (F32) {
       bf16x4 hi, lo;
 #pragma unroll
@@ -385,7 +390,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
   if (nunits > 64) load_block(1);
   to_ring(0, cur);
   form_read(0, cur);
-  static_for<0, UA + UB>([&](auto k) { form_block(k, 0); });
+  static_for<0, UA + UB>([&](auto k) {
+    form_read_block(k, 0, cur);
+    form_block(k, 0);
+  });
 
   // masked rows start their scores at -inf (p = 0); a scale of 0 gets a tiny
   // factor instead, so that -inf times it stays -inf (dS carries the scale)
@@ -445,7 +453,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
       for (int s = 0; s < PK; ++s) bias[c][s] = kw <= ut[s] && kw >= lo2[s] ? lse2[s] : INFINITY;
     }
     const int nbuf = (st + 1) & 1;
-    auto sinit = [&](int e) {
+    auto sinit = [&](int, int e) {
       constexpr int kSub = 16 / PK;  // registers per unit
       const int row = (8 * (e >> 2) + (e & 3)) % R + 4 * half;
       return row < ilo[e / kSub] ? smask : 0.f;
@@ -460,6 +468,13 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
       constexpr int i = decltype(ii)::value, NB = UA + UB, T4 = C::T4;
       constexpr int first = T4 / 4;
       if constexpr (i == 0) form_read(st + 1, nx1);
+      static_for<0, NB>([&](auto kk) {
+        constexpr int k = decltype(kk)::value;
+        constexpr int at = first + k * (T4 - first) / NB;  // item that forms block k
+        // wide rows: two items earlier its source is read (all at once they
+        // take the registers that the fragments leave)
+        if constexpr ((DK > 256 ? (at > 2 ? at - 2 : 0) : 0) == i) form_read_block(kk, st + 1, nx1);
+      });
       static_for<0, NB>([&](auto kk) {
         constexpr int k = decltype(kk)::value;
         if constexpr (first + k * (T4 - first) / NB == i) form_block(kk, nbuf);
@@ -537,13 +552,22 @@ int dkv2_pieces(int64_t blocks, int64_t steps, int64_t cus, int64_t room) {
   return best;
 }
 
+template <int DK, int DV, int SETS, int PK, bool F32, int KB0, int KBN, int VBN>
+hipError_t launch_dkv2_slice(const BwdParams& p, const Dkv2Geo& geo, hipStream_t stream) {
+  const size_t lds = Dkv2Lds<DK, DV, PK, F32>::bytes(geo.ring);
+  auto kern = bwd_dkv2_kernel<DK, DV, SETS, PK, F32, KB0, KBN, VBN>;
+  hipError_t e = set_lds_limit((const void*)kern, lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(geo.nblocks), dim3(256), lds, stream, p, geo);
+  return hipGetLastError();
+}
+
 template <int DK, int DV, int SETS, int PK, bool F32>
 hipError_t launch_dkv2_t(const BwdParams& p, size_t scratch_bytes, hipStream_t stream) {
-  using L = Dkv2Lds<DK, DV, PK, F32>;
   constexpr int KB = 128 * SETS;
   Dkv2Geo geo{};
   geo.nr = PK > 1 ? 1 : (p.ws + 31) / 32;
-  geo.ring = geo.nr <= 2 ? 64 : 128;
+  geo.ring = DK > 256 ? 32 : geo.nr <= 2 ? 64 : 128;
   geo.kblocks = (p.tokens + KB - 1) / KB;
   const int64_t blocks = (int64_t)geo.kblocks * p.hk;
   const int64_t per = dkv2_piece_bytes(p.tokens, p.hk, DK, DV);
@@ -553,12 +577,15 @@ hipError_t launch_dkv2_t(const BwdParams& p, size_t scratch_bytes, hipStream_t s
   geo.splits = F32 ? 1 : dkv2_pieces(blocks, queries * p.group * geo.nr / PK, device_cu_count(),
                                      p.dkv2s ? (int64_t)scratch_bytes / per : 1);
   geo.nblocks = (int)(blocks * geo.splits);
-  const size_t lds = L::bytes(geo.ring);
-  auto kern = bwd_dkv2_kernel<DK, DV, SETS, PK, F32>;
-  hipError_t e = set_lds_limit((const void*)kern, lds);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3(geo.nblocks), dim3(256), lds, stream, p, geo);
-  e = hipGetLastError();
+  hipError_t e;
+  if constexpr (DK > 256) {
+    // accumulators of 512 + 256 columns take 384 registers: two launches
+    constexpr int kFirst = 4;
+    e = launch_dkv2_slice<DK, DV, SETS, PK, F32, 0, kFirst, DV / 32>(p, geo, stream);
+    if (e == hipSuccess) e = launch_dkv2_slice<DK, DV, SETS, PK, F32, kFirst, DK / 32 - kFirst, 0>(p, geo, stream);
+  } else {
+    e = launch_dkv2_slice<DK, DV, SETS, PK, F32, 0, DK / 32, DV / 32>(p, geo, stream);
+  }
   if (e != hipSuccess || geo.splits == 1) return e;
   const int64_t threads = (int64_t)p.tokens * p.hk * ((DK + DV) / 4);
   hipLaunchKernelGGL(bwd_dkv2_sum_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p, geo.splits);
@@ -589,7 +616,11 @@ hipError_t launch_bwd_dkv2_mfma(const BwdParams& p, size_t scratch_bytes, hipStr
     return p.d == 64 ? launch_dkv2_pk<64, 64, 2, true>(p, scratch_bytes, stream)
                      : launch_dkv2_pk<128, 128, 1, true>(p, scratch_bytes, stream);
   }
-  if (p.ws > (p.d > 128 ? 64 : 128)) return hipErrorNotSupported;
+  if (p.ws > (p.d > 256 ? 32 : p.d > 128 ? 64 : 128)) return hipErrorNotSupported;
+  if (p.d == 512) {
+    if (p.ws <= 16) return launch_dkv2_t<512, 256, 1, 2, false>(p, scratch_bytes, stream);
+    return launch_dkv2_t<512, 256, 1, 1, false>(p, scratch_bytes, stream);
+  }
   if (p.d == 256)
     return p.dv == 256 ? launch_dkv2_pk<256, 256, 1>(p, scratch_bytes, stream)
                        : launch_dkv2_pk<256, 128, 1>(p, scratch_bytes, stream);

@@ -1217,7 +1217,7 @@ bool bwd_mfma_ok(const BwdParams& p) {
   if (!p.mfma) return false;
   if (p.f32 && (p.d != p.dv || (p.d != 64 && p.d != 128) || !p.k2s || !p.v2s)) return false;
   const bool narrow = (p.d == 64 || p.d == 128) && (p.dv == 64 || p.dv == 128);
-  if (!narrow && !(p.d == 256 && (p.dv == 128 || p.dv == 256))) return false;
+  if (!narrow && !(p.d == 256 && (p.dv == 128 || p.dv == 256)) && !(p.d == 512 && p.dv == 256)) return false;
   const int64_t st[] = {p.q_st, p.q_sh, p.k_st, p.k_sh, p.v_st, p.v_sh, p.do_st, p.do_sh};
   for (int64_t s : st)
     if (s % 8) return false;
@@ -1232,7 +1232,7 @@ bool bwd_mfma_ok(const BwdParams& p) {
 }
 
 hipError_t launch_bwd_dq_mfma(const BwdParams& p, hipStream_t stream) {
-  if (!bwd_mfma_ok(p)) return hipErrorNotSupported;
+  if (!bwd_mfma_ok(p) || p.d > 256) return hipErrorNotSupported;
   const BwdGeo geo = base_geo(p);
   if (p.f32) {
     if (p.ws > 32) return hipErrorNotSupported;  // fp32: one 32-row group of short keys
@@ -1242,7 +1242,7 @@ hipError_t launch_bwd_dq_mfma(const BwdParams& p, hipStream_t stream) {
 }
 
 hipError_t launch_bwd_dkv1_mfma(const BwdParams& p, hipStream_t stream) {
-  if (!bwd_mfma_ok(p)) return hipErrorNotSupported;
+  if (!bwd_mfma_ok(p) || p.d > 256) return hipErrorNotSupported;
   const BwdGeo geo = base_geo(p);
   if (p.f32) {
     if (p.ws > 32) return hipErrorNotSupported;  // fp32: one 32-row group of short keys
@@ -1251,7 +1251,7 @@ hipError_t launch_bwd_dkv1_mfma(const BwdParams& p, hipStream_t stream) {
   return by_widths<true>(p, [&](auto dk, auto dv) { return launch_dkv1_d<decltype(dk)::value, decltype(dv)::value>(p, geo, stream); });
 }
 bool bwd_dk1_fused_ok(const BwdParams& p) {
-  return bwd_mfma_ok(p) && p.ws <= (p.f32 ? 32 : 64);
+  return bwd_mfma_ok(p) && p.d <= 256 && p.ws <= (p.f32 ? 32 : 64);
 }
 
 hipError_t launch_bwd_dk1_sum(const BwdParams& p, hipStream_t stream) {

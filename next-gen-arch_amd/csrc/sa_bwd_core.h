@@ -112,30 +112,34 @@ __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 3
 
 // F32: every operand as hi + lo bf16 terms (split_bf16), each product on three
 // term pairs; the lo tile rows follow the 32 (TR) hi rows of each tile.
-// TR: rows of a tile in LDS (32, or more where waves read it at row offsets).
-template <int DK, int DV, int SETS, bool F32, int TR = 32>
+// KB0, KBN: the 32-column blocks of the score width whose ak is accumulated;
+// VBN: the blocks of av (DV / 32, or 0: no av).  A width whose accumulators do
+// not fit the registers takes one launch per slice, which forms the scores anew.
+template <int DK, int DV, int SETS, bool F32, int KB0 = 0, int KBN = DK / 32, int VBN = DV / 32>
 struct BwdCore {
+  static constexpr int TR = 32;                            // rows of a tile
   static constexpr int WK = 2 * DK, WV = 2 * DV;           // bytes of a tile row
   static constexpr int TK = TR * WK * (F32 ? 2 : 1);       // bytes of a K tile (hi, then lo rows)
   static constexpr int TV = TR * WV * (F32 ? 2 : 1);
   static constexpr int LOK = TR * WK, LOV = TR * WV;       // offset of the lo rows
   // items read ahead (with one set an item lasts one MFMA: further ahead)
   static constexpr int kAhead = F32 ? 3 : SETS == 1 ? 5 : DK + DV >= 256 ? 3 : 4;
-  static constexpr int T1 = DK / 16, T2 = DV / 16, T3 = DV / 16, T4 = DK / 16;
+  static constexpr int T1 = DK / 16, T2 = DV / 16, T3 = 2 * VBN, T4 = 2 * KBN;
+  static_assert(VBN == 0 || VBN == DV / 32, "all of av or none");
   static constexpr int NT = T1 + T2 + T3 + T4;
   static constexpr int NX = F32 ? 2 : 1;                   // terms per operand
 
   bf16x8 kx[SETS][T1], vx[SETS][T2];
   bf16x8 kxl[F32 ? SETS : 1][F32 ? T1 : 1], vxl[F32 ? SETS : 1][F32 ? T2 : 1];
-  floatx16 ak[SETS][DK / 32], av[SETS][DV / 32];
+  floatx16 ak[SETS][KBN], av[SETS][VBN ? VBN : 1];
 
   __device__ __forceinline__ void clear() {
 #pragma unroll
     for (int c = 0; c < SETS; ++c) {
 #pragma unroll
-      for (int i = 0; i < DK / 32; ++i) ak[c][i] = floatx16{};
+      for (int i = 0; i < KBN; ++i) ak[c][i] = floatx16{};
 #pragma unroll
-      for (int i = 0; i < DV / 32; ++i) av[c][i] = floatx16{};
+      for (int i = 0; i < VBN; ++i) av[c][i] = floatx16{};
     }
   }
 
@@ -185,7 +189,8 @@ struct BwdCore {
       constexpr bool isk = I >= T1 + T2 + T3;
       constexpr int D = isk ? DK : DV, W = 2 * D;
       constexpr int s = isk ? I - T1 - T2 - T3 : I - T1 - T2;
-      constexpr int t = s / (D / 32), db = s % (D / 32);
+      constexpr int NB = isk ? KBN : VBN ? VBN : 1;
+      constexpr int t = s / NB, db = s % NB + (isk ? KB0 : 0);
       constexpr int xm = W >= 256 ? 64 * (db & 3) : 64 * db;
       constexpr int off = (W >= 256 ? 256 * (db >> 2) : 0) + 16 * t * W;
       const uint32_t a = (isk ? ad.kc : ad.vc) ^ xm, b = a ^ 32;
@@ -207,8 +212,8 @@ struct BwdCore {
       return __builtin_bit_cast(bf16x8, u32x4{f.a[0], f.a[1], f.b[0], f.b[1]});
     }
   }
-  // One step for the sets in ACT (a bit mask).  sinit(e): start value of score
-  // register e (0, or the value that masks it) when `masked`.  prob(c, e, s):
+  // One step for the sets in ACT (a bit mask).  sinit(c, e): start value of score
+  // register e of set c (0, or the value that masks it) when `masked`.  prob(c, e, s):
   // the probability of register e of set c; grad(c, e, p, dp): its dS.
   // fill(item): the caller's work beside item 0 .. T4-1 of phase 4.
   template <int ACT, typename SI, typename PF, typename GF, typename FF>
@@ -223,7 +228,7 @@ struct BwdCore {
       constexpr int c = decltype(cc)::value;
       if (masked) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[c][e] = sinit(e);
+        for (int e = 0; e < 16; ++e) s[c][e] = sinit(c, e);
         mfma_v<true>(s[c], h, kx[c][0]);
       } else {
         mfma_v0(s[c], h, kx[c][0]);
@@ -247,8 +252,8 @@ struct BwdCore {
         constexpr int c = decltype(cc)::value, cl = F32 ? c : 0;
         if constexpr ((ACT >> c) & 1) {
           // first use of vector results: the start scores, the packed P and dS.
-          // (fp32: fragments may be moved out of accumulation registers)
-          constexpr bool nop = F32 || I == 0 || I == T1 + T2 || I == T1 + T2 + T3;
+          // (fp32 and width 512: fragments are moved out of accumulation registers)
+          constexpr bool nop = F32 || DK > 256 || I == 0 || I == T1 + T2 || I == T1 + T2 + T3;
           if constexpr (I < T1) {
             if constexpr (I == 0) first(cc, h);
             else mfma_v<nop>(s[c], h, kx[c][I]);
@@ -266,9 +271,19 @@ struct BwdCore {
             }
           } else {
             constexpr bool isk = I >= T1 + T2 + T3;
-            constexpr int D = isk ? DK : DV;
+            constexpr int NB = isk ? KBN : VBN ? VBN : 1;
             constexpr int q = isk ? I - T1 - T2 - T3 : I - T1 - T2;
-            constexpr int t = q / (D / 32), db = q % (D / 32);
+            constexpr int t = q / NB, db = q % NB;
+            if constexpr (VBN == 0 && I == T1 + T2) {  // no av phase to form dS beside
+              asm volatile("s_nop 15" : "+v"(dp[c]));
+#pragma unroll
+              for (int e = 0; e < 16; ++e) dp[c][e] = grad(c, e, s[c][e], dp[c][e]);
+#pragma unroll
+              for (int i = 0; i < 8; ++i) {
+                if constexpr (F32) pack_bf16_split(dp[c][2 * i], dp[c][2 * i + 1], pk[c][i], pl[cl][i]);
+                else pk[c][i] = pack_bf16(dp[c][2 * i], dp[c][2 * i + 1]);
+              }
+            }
             const bf16x8 b = __builtin_bit_cast(bf16x8, u32x4{pk[c][4 * t], pk[c][4 * t + 1], pk[c][4 * t + 2], pk[c][4 * t + 3]});
             const bf16x8 bl = __builtin_bit_cast(bf16x8, u32x4{pl[cl][4 * t], pl[cl][4 * t + 1], pl[cl][4 * t + 2], pl[cl][4 * t + 3]});
             floatx16& acc = isk ? ak[c][isk ? db : 0] : av[c][isk ? 0 : db];
@@ -299,8 +314,8 @@ struct BwdCore {
                 s[c][2 * i + 1] = prob(c, 2 * i + 1, s[c][2 * i + 1]);
               }
             });
-            if constexpr (I > T1) pack(std::integral_constant<int, I - T1 - 1>{});
-            if constexpr (I == T1 + T2 - 1) pack(std::integral_constant<int, T2 - 1>{});
+            if constexpr (VBN > 0 && I > T1) pack(std::integral_constant<int, I - T1 - 1>{});
+            if constexpr (VBN > 0 && I == T1 + T2 - 1) pack(std::integral_constant<int, T2 - 1>{});
             __builtin_amdgcn_sched_barrier(0);
           } else if constexpr (I >= T1 + T2 && I < T1 + T2 + T3) {
             if constexpr (I == T1 + T2) mfma_settle(dp[c]);

@@ -1,0 +1,33 @@
+"""dq / dk1 / dv1 pass at the edges of its workgroups: groups that divide a
+workgroup's units, are divided by them or neither, last units past the tokens,
+short windows at the 16-key units, and sequences that end inside a workgroup.
+All five gradients against the portable kernels (same rounding points, another
+order of the fp32 sums: 2e-2 of the largest gradient) and for repeatability."""
+
+import pytest
+import torch
+
+from helpers import rand_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,hq,hk,d,dv,ws,wl", [
+    (131, 4, 1, 512, 256, 32, 40),
+    (67, 3, 1, 512, 256, 17, 300),
+    (90, 2, 2, 512, 256, 16, 33),
+    (53, 8, 1, 512, 256, 1, 7),
+])
+def test_dq_block_edges(cuda, n, hq, hk, d, dv, ws, wl):
+    from archlab_amd import simplicial_varlen_attention
+    x = [t[0].to(cuda) for t in rand_inputs(1, n, hq, hk, d, dv, seed=n + ws)]
+    cu = torch.tensor([0, 1, n // 3, n // 3 + 5, n], dtype=torch.int32, device=cuda)
+    dout = torch.randn(n, hq, dv, generator=torch.Generator().manual_seed(n)).to(x[0].dtype).to(cuda)
+    runs = []
+    for kernel in ("auto", "auto", "generic"):
+        xd = [t.clone().requires_grad_(True) for t in x]
+        simplicial_varlen_attention(*xd, cu, ws, wl, kernel=kernel).backward(dout)
+        runs.append([t.grad.float() for t in xd])
+    for name, a, a2, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), *runs):
+        assert torch.isfinite(a).all() and torch.equal(a, a2), name
+        assert (a - b).abs().max().item() <= 2e-2 * max(b.abs().max().item(), 1.0), name
