@@ -17,6 +17,12 @@ pytestmark = pytest.mark.gpu
     (67, 3, 1, 512, 256, 17, 300),
     (90, 2, 2, 512, 256, 16, 33),
     (53, 8, 1, 512, 256, 1, 7),
+    (131, 16, 4, 128, 128, 16, 40),
+    (67, 3, 1, 128, 128, 7, 300),
+    (90, 2, 2, 128, 128, 16, 33),
+    (53, 24, 1, 128, 128, 1, 7),
+    (131, 4, 4, 64, 64, 16, 70),
+    (75, 12, 2, 64, 64, 13, 90),
 ])
 def test_dq_block_edges(cuda, n, hq, hk, d, dv, ws, wl):
     from archlab_amd import simplicial_varlen_attention
