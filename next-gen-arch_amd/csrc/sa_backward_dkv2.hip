@@ -613,8 +613,14 @@ hipError_t launch_bwd_dkv2_mfma(const BwdParams& p, size_t scratch_bytes, hipStr
   if (!bwd_mfma_ok(p)) return hipErrorNotSupported;
   if (p.f32) {
     if (p.ws > 32) return hipErrorNotSupported;
-    return p.d == 64 ? launch_dkv2_pk<64, 64, 2, true>(p, scratch_bytes, stream)
-                     : launch_dkv2_pk<128, 128, 1, true>(p, scratch_bytes, stream);
+    if (p.d == 128) return launch_dkv2_pk<128, 128, 1, true>(p, scratch_bytes, stream);
+    // fp32 walks are not cut into pieces: where blocks of 128 keys all run at
+    // once, two sets per wave only lengthen the walks (2048 tokens, 8 / 8 heads,
+    // windows 32 x 256, forward + backward: 1.63 ms with two, 1.13 with one; 6000
+    // tokens, 376 such blocks: 2.47 ms with two)
+    const int64_t blocks = ((int64_t)p.tokens + 127) / 128 * p.hk;
+    return blocks <= device_cu_count() ? launch_dkv2_pk<64, 64, 1, true>(p, scratch_bytes, stream)
+                                       : launch_dkv2_pk<64, 64, 2, true>(p, scratch_bytes, stream);
   }
   if (p.ws > (p.d > 256 ? 32 : p.d > 128 ? 64 : 128)) return hipErrorNotSupported;
   if (p.d == 512) {

@@ -25,7 +25,10 @@ pytestmark = pytest.mark.gpu
     (200, 4, 1, 256, 64, 100, "bf16"),   # ... two row groups in one walk
     (150, 2, 1, 64, 128, 140, "bf16"),   # four row groups
     (257, 6, 2, 128, 8, 30, "f32"),
-    (129, 3, 3, 64, 16, 129, "f32"),
+    (129, 3, 3, 64, 16, 129, "f32"),     # width 64: 128-key blocks where they all run at once
+    (200, 4, 2, 64, 32, 70, "f32"),
+    (131, 4, 2, 64, 8, 40, "f32"),
+    (257, 129, 129, 64, 32, 40, "f32"),  # ... 256-key blocks past that
 ])
 def test_dkv2_step_edges(cuda, n, hq, hk, d, ws, wl, dtype):
     from archlab_amd import simplicial_varlen_attention
