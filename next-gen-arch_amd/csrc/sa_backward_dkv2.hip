@@ -33,6 +33,7 @@
 // leave CUs idle in the last wave of workgroups: each piece writes fp32 sums
 // that bwd_dkv2_sum_kernel adds in piece order (no atomics).
 #include "sa_bwd_core.h"
+#include "sa_bwd_walk.h"
 #include "sa_launch.h"
 #include "sa_backward.h"
 
@@ -181,16 +182,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
   }
 
   // Unit state, carried from step to step (no divisions in the step loop).
-  struct Unit {
-    int t, h, r;  // h: head within the group
-  };
-  auto advance = [&](Unit u) {
-    if (++u.r == nr) {
-      u.r = 0;
-      if (++u.h == G) u.h = 0, ++u.t;
-    }
-    return u;
-  };
+  using Unit = WalkUnit;
+  auto advance = [&](Unit u) { return walk_next(u, G, nr); };
   auto after = [&](Unit u) {  // the first unit of the next step
 #pragma unroll
     for (int s = 0; s < PK; ++s) u = advance(u);
@@ -199,8 +192,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
 
   // Stage slot st % 2: per unit its q, dout, k1_t and v1_t rows end to end
   // (lanes past them re-fetch the first segment into the unused tail); units
-  // past the walk stage whatever follows its last query, or that query again
-  // at the end of the tensors (their probabilities are zero).  A lane's tensor
+  // past the walk stage its last unit's rows again (walk_moves: nothing past
+  // them is read, and their zero probabilities multiply rows that the walk
+  // multiplies anyway).  A lane's tensor
   // is fixed by its byte offset: its row pointer is carried from unit to unit
   // (next head: + one head stride; next query: + the rest of a token stride),
   // in place of four row addresses and a selection per step.
@@ -228,11 +222,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
 #pragma unroll
       for (int k = 0; k < SI; ++k) dma16(dptr[k], stage + ((st & 1) * PK + s) * SS + 1024 * k);
       const Unit y = advance(dunit);
-      if (y.h != dunit.h || y.t != dunit.t) {  // (row groups of a head share its rows)
-        if (y.t == dunit.t || y.t <= last) {
+      if (walk_moves(dunit, y, st * PK + s, nunits, PK)) {
 #pragma unroll
-          for (int k = 0; k < SI; ++k) dptr[k] += (int64_t)(y.t == dunit.t ? dhead[k] : dtok[k]) * 16;
-        }
+        for (int k = 0; k < SI; ++k) dptr[k] += (int64_t)(y.t == dunit.t ? dhead[k] : dtok[k]) * 16;
       }
       dunit = y;
     }
