@@ -86,11 +86,14 @@ enum { SA_INDEX_I32 = 0, SA_INDEX_I64 = 1 };
 
 enum {
   SA_FLAG_FORCE_GENERIC = 1, /* use the portable (non-MFMA) kernel; for cross-checks */
-  /* sa_prefill_bwd only: compute dk1 in a pass of its own instead of from
-   * partials written by the dq pass.  The workspace then holds no dk1
-   * partials (those take 16-17.5x the bytes of q per 32 keys of short
-   * window); the backward runs one more recomputation pass (about 20 % more
-   * time at the benchmark shape). */
+  /* sa_prefill_bwd only, for callers short of memory: the workspace holds no
+   * dk1 / dv1 partials (those take 16-17.5x the bytes of q per 32 keys of
+   * short window).  dk1 is computed in a pass of its own, one more
+   * recomputation pass (about 20 % more time at the benchmark shape); bf16
+   * calls with at most 16 short keys keep the pass with partials, in phases over
+   * the queries, where the space of the dk2 / dv2 pieces holds a phase that
+   * fills half of the GPU.
+   * At head_dim 512 dq, dk1 and dv1 run on the portable kernels. */
   SA_FLAG_SEPARATE_DK1 = 2,
   /* Paged calls whose windows are consecutive blocks (contiguous decodes):
    * token i is sequence i at position long_window - 1.  Position p of sequence

@@ -27,10 +27,16 @@
 // Its partials take less than the scratch that the dk1 partials had.  Two sets
 // of 128 + 128 columns spill 73 registers, outside the unmasked steps.
 //
-// Partials past the workspace: the blocks run in phases, each followed by the
-// sum of the keys it completes; a phase starts with the blocks of the last
-// unfinished keys again.
+// Partials past the workspace: the blocks run in phases (dq_phase), each
+// followed by the sum of the keys it completes; a phase starts with the blocks of
+// the last unfinished keys again.  At widths of 64 and 128, where passes without
+// partials stand beside this one, only where a phase takes more than half of the
+// CUs.  Against those passes, backward with 16 short keys, width 128: phases of 512
+// workgroups (2048 tokens, 32 / 1 heads, 9 phases) 19.1 -> 14.9 ms, of 256 (4096,
+// 16 / 1, 18 phases) 11.0 -> 10.2; of 128 (2048, 16 / 1) 8.9 -> 9.0, of 88 (1500, 8
+// / 1) 5.0 -> 5.2.
 #include "sa_bwd_core.h"
+#include "sa_bwd_walk.h"
 #include "sa_launch.h"
 #include "sa_backward.h"
 
@@ -43,7 +49,6 @@ namespace {
 struct DqGeo {
   int nblocks;  // workgroups of the launch
   int b0, nb;   // blocks [b0, b0 + nb) of every KV head
-  int blocks;   // blocks per KV head
   int nr;       // 32-row groups of short keys (1 with PK > 1)
   int nrows;    // short-key rows of a block's partial
   float* part;  // [hk][nb][nr][nrows][DK + DV]
@@ -351,21 +356,19 @@ hipError_t launch_dq_t(const BwdParams& p, size_t scratch_bytes, hipStream_t str
   DqGeo geo{};
   geo.nr = PK > 1 ? 1 : (p.ws + 31) / 32;
   geo.nrows = R - 1 + block_queries(U, p.group);
-  geo.blocks = (int)(((int64_t)p.tokens * p.group + U - 1) / U);
   geo.part = p.dkv2s;
   const int64_t bytes = (int64_t)p.hk * geo.nr * geo.nrows * (DK + DV) * sizeof(float);  // of a block of every KV head
   const int64_t cap = (int64_t)(scratch_bytes / bytes);
   const int reach = R - 1 + 32 * (geo.nr - 1);  // queries after its own that a key waits for
-  if (cap < geo.blocks && cap < 4 * (((int64_t)reach * p.group + U - 1) / U + 1)) return hipErrorNotSupported;
-  int j0 = 0;
-  while (j0 < p.tokens) {
-    geo.b0 = (int)((int64_t)j0 * p.group / U);
-    geo.nb = (int)std::min<int64_t>(cap, geo.blocks - geo.b0);
+  // (score width 512: the portable kernels otherwise)
+  const int64_t least = DK > 256 ? 1 : device_cu_count() / 2 / p.hk + 1;
+  if (!dq_phases_pay(p.tokens, p.group, U, reach, cap, least)) return hipErrorNotSupported;
+  for (int j0 = 0; j0 < p.tokens;) {
+    const DqPhase ph = dq_phase(j0, p.tokens, p.group, U, reach, cap);
+    geo.b0 = ph.b0;
+    geo.nb = ph.nb;
     geo.nblocks = geo.nb * p.hk;
-    const bool end = geo.b0 + geo.nb == geo.blocks;
-    // the phase completes the queries before tend, and the keys `reach` before it
-    const int tend = (int)((int64_t)(geo.b0 + geo.nb) * U / p.group);
-    const int j1 = end ? p.tokens : tend - reach;
+    const int j1 = ph.j1;
     hipError_t e;
     if constexpr (DK > 256) {
       // accumulators of 512 + 256 columns take 384 registers: two launches

@@ -1,10 +1,11 @@
-// Walk of the dk2 / dv2 pass over its units: query t, head h of the KV group,
-// 32-row group r of t's short keys, in ascending (t, h, r).  constexpr, so that
-// the kernel and host checks run the same steps.
+// Index walks of the backward passes, constexpr so that the kernels, their
+// launches and host checks run the same steps.
 #pragma once
 
 namespace sa {
 
+// dk2 / dv2 pass: units in ascending (query t, head h of the KV group, 32-row
+// group r of t's short keys).
 struct WalkUnit {
   int t, h, r;  // h: head within the group
 };
@@ -24,6 +25,32 @@ constexpr WalkUnit walk_next(WalkUnit u, int group, int nr) {
 // (One unit per step: nothing is staged after the last.)
 constexpr bool walk_moves(WalkUnit u, WalkUnit y, int i, int n, int pk) {
   return (y.h != u.h || y.t != u.t) && (pk == 1 || i + 1 < n);
+}
+
+
+// dq / dk1 / dv1 pass: blocks of U consecutive units (t, h), whose partials may
+// take more space than there is (room for `cap` blocks).  It then runs in
+// phases, blocks [b0, b0 + nb) each, followed by the sums of the keys [j0, j1)
+// that the phase completes: a key waits for the queries up to `reach` after its
+// own, so the next phase starts with the blocks of the last `reach` queries.
+struct DqPhase {
+  int b0, nb, j0, j1;
+};
+
+constexpr DqPhase dq_phase(int j0, int tokens, int group, int U, int reach, long long cap) {
+  const long long blocks = ((long long)tokens * group + U - 1) / U;
+  const long long b0 = (long long)j0 * group / U;
+  const long long nb = cap < blocks - b0 ? cap : blocks - b0;
+  const int tend = (int)((b0 + nb) * U / group);  // queries before it are complete
+  return {(int)b0, (int)nb, j0, b0 + nb == blocks ? tokens : tend - reach};
+}
+
+// Whether the pass runs, in one phase or in phases of at least `least` blocks of
+// which about a quarter at most is repeated by the next one.
+constexpr bool dq_phases_pay(int tokens, int group, int U, int reach, long long cap, long long least) {
+  const long long blocks = ((long long)tokens * group + U - 1) / U;
+  const long long repeated = ((long long)reach * group + U - 1) / U + 1;
+  return cap >= blocks || (cap >= 4 * repeated && cap >= least);
 }
 
 }  // namespace sa

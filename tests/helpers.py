@@ -88,3 +88,40 @@ def paged_batch(lengths, kv_heads, dim, block_size, dtype, hnd=False, seed=0, de
     if hnd:
         caches = [c.transpose(2, 3) for c in caches]
     return [c.to(device) for c in caches], table.to(device), dense
+
+
+def backward_grads(x, dout, cu, ws, wl, flags=0, scratch=None):
+    """dq, dk1, dk2, dv1, dv2 of [T, H, *] tensors of any layout through the C ABI.
+    ``scratch`` (a list): receives the workspace bytes past the delta and dlse rows."""
+    import ctypes
+
+    from archlab_amd import _native
+    from archlab_amd.architectures.simplicial_attention import _prefill
+    lib, dev = _native.load(), x[0].device
+    dense = [t.contiguous() for t in x]
+    out, lse = _prefill(*dense, ws, wl, 0.3, cu, cu.numel() - 1, 0, True, 
+                        "generic" if flags & _native.SA_FLAG_FORCE_GENERIC else "auto")
+    grads = [torch.empty_like(t) for t in dense]
+    q, k1, k2, v1, v2 = x
+    dq, dk1, dk2, dv1, dv2 = grads
+    fwd = _native.PrefillArgs(
+        q=q.data_ptr(), k1=k1.data_ptr(), k2=k2.data_ptr(), v1=v1.data_ptr(), v2=v2.data_ptr(), out=out.data_ptr(),
+        lse=lse.data_ptr(), cu_seqlens=cu.data_ptr(), q_stride_t=q.stride(0), q_stride_h=q.stride(1),
+        k_stride_t=k1.stride(0), k_stride_h=k1.stride(1), v_stride_t=v1.stride(0), v_stride_h=v1.stride(1),
+        o_stride_t=out.stride(0), o_stride_h=out.stride(1), lse_stride_t=lse.stride(0), num_seqs=cu.numel() - 1,
+        total_tokens=q.shape[0], heads_q=q.shape[1], heads_kv=k1.shape[1], head_dim=q.shape[2],
+        value_dim=v1.shape[2], short_window=ws, long_window=wl, scale=0.3, dtype=_native.dtype_code(q.dtype),
+        flags=flags)
+    args = _native.PrefillBwdArgs(
+        fwd=fwd, dout=dout.data_ptr(), do_stride_t=dout.stride(0), do_stride_h=dout.stride(1), dq=dq.data_ptr(),
+        dq_stride_t=dq.stride(0), dq_stride_h=dq.stride(1), dk1=dk1.data_ptr(), dk2=dk2.data_ptr(),
+        dk_stride_t=dk1.stride(0), dk_stride_h=dk1.stride(1), dv1=dv1.data_ptr(), dv2=dv2.data_ptr(),
+        dv_stride_t=dv1.stride(0), dv_stride_h=dv1.stride(1))
+    nbytes = lib.sa_prefill_bwd_workspace_bytes(ctypes.byref(args))
+    if scratch is not None:
+        scratch.append(nbytes - 2 * ((q.shape[0] * q.shape[1] * 4 + 255) // 256 * 256))
+    work = torch.empty(nbytes + 256, device=dev, dtype=torch.uint8)
+    _native.check(lib.sa_prefill_bwd(ctypes.byref(args), (work.data_ptr() + 255) & ~255, nbytes,
+                                     _native.stream_handle(dev)))
+    torch.cuda.synchronize()
+    return grads

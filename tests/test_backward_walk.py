@@ -56,39 +56,6 @@ def test_staged_rows_stay_inside_the_walk(tmp_path):
     assert run.returncode == 0, run.stdout
 
 
-def _grads(x, dout, cu, ws, wl):
-    """dq, dk1, dk2, dv1, dv2 of tensors of any layout through the C ABI."""
-    import ctypes
-
-    import torch
-    from archlab_amd import _native
-    from archlab_amd.architectures.simplicial_attention import _prefill
-    lib, dev = _native.load(), x[0].device
-    dense = [t.contiguous() for t in x]
-    out, lse = _prefill(*dense, ws, wl, 0.3, cu, cu.numel() - 1, 0, True, "auto")
-    grads = [torch.empty_like(t) for t in dense]
-    q, k1, k2, v1, v2 = x
-    dq, dk1, dk2, dv1, dv2 = grads
-    fwd = _native.PrefillArgs(
-        q=q.data_ptr(), k1=k1.data_ptr(), k2=k2.data_ptr(), v1=v1.data_ptr(), v2=v2.data_ptr(), out=out.data_ptr(),
-        lse=lse.data_ptr(), cu_seqlens=cu.data_ptr(), q_stride_t=q.stride(0), q_stride_h=q.stride(1),
-        k_stride_t=k1.stride(0), k_stride_h=k1.stride(1), v_stride_t=v1.stride(0), v_stride_h=v1.stride(1),
-        o_stride_t=out.stride(0), o_stride_h=out.stride(1), lse_stride_t=lse.stride(0), num_seqs=cu.numel() - 1,
-        total_tokens=q.shape[0], heads_q=q.shape[1], heads_kv=k1.shape[1], head_dim=q.shape[2],
-        value_dim=v1.shape[2], short_window=ws, long_window=wl, scale=0.3, dtype=_native.dtype_code(q.dtype))
-    args = _native.PrefillBwdArgs(
-        fwd=fwd, dout=dout.data_ptr(), do_stride_t=dout.stride(0), do_stride_h=dout.stride(1), dq=dq.data_ptr(),
-        dq_stride_t=dq.stride(0), dq_stride_h=dq.stride(1), dk1=dk1.data_ptr(), dk2=dk2.data_ptr(),
-        dk_stride_t=dk1.stride(0), dk_stride_h=dk1.stride(1), dv1=dv1.data_ptr(), dv2=dv2.data_ptr(),
-        dv_stride_t=dv1.stride(0), dv_stride_h=dv1.stride(1))
-    nbytes = lib.sa_prefill_bwd_workspace_bytes(ctypes.byref(args))
-    work = torch.empty(nbytes + 256, device=dev, dtype=torch.uint8)
-    _native.check(lib.sa_prefill_bwd(ctypes.byref(args), (work.data_ptr() + 255) & ~255, nbytes,
-                                     _native.stream_handle(dev)))
-    torch.cuda.synchronize()
-    return grads
-
-
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("layout", ["token", "head"])
@@ -98,7 +65,7 @@ def test_rows_past_the_tensors_are_not_used(cuda, n, hq, hk, ws, layout, dtype):
     heads of a token or the tokens of a head adjacent: the gradients are
     those of separate tensors, bit for bit."""
     import torch
-    from helpers import rand_inputs
+    from helpers import backward_grads, rand_inputs
     dt = torch.bfloat16 if dtype == "bf16" else torch.float32
     x = [t[0] for t in rand_inputs(1, n, hq, hk, 64, seed=n, dtype=dt, device=cuda)]
     x.append(torch.randn(n, hq, 64, generator=torch.Generator().manual_seed(n)).to(dt).to(cuda))  # dout
@@ -114,8 +81,8 @@ def test_rows_past_the_tensors_are_not_used(cuda, n, hq, hk, ws, layout, dtype):
         view.copy_(t)
         return view
 
-    want = _grads(x[:5], x[5], cu, ws, 20)
+    want = backward_grads(x[:5], x[5], cu, ws, 20)
     y = [front(t) for t in x]
-    got = _grads(y[:5], y[5], cu, ws, 20)
+    got = backward_grads(y[:5], y[5], cu, ws, 20)
     for name, a, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), got, want):
         assert torch.isfinite(b).all() and torch.equal(a, b), name
