@@ -61,8 +61,9 @@ struct DqLds {
   static constexpr int CS = 32 * KBN < 128 || DV < 128 ? 64 : 128;  // columns per epilogue slab
   static constexpr int MAIN = 2 * TAB > S * 32 * CS * 4 ? 2 * TAB : S * 32 * CS * 4;
   static constexpr int ROWS = U * 2 * (DK + DV);                // q and dout rows of the units
+  static constexpr int LO1 = U * 4;                             // first short key of the units
   static constexpr int DQS = U * 32 * KBN * 4;                  // dq sums over row groups
-  static constexpr size_t bytes(int nr) { return MAIN + ROWS + (nr > 1 ? DQS : 0); }
+  static constexpr size_t bytes(int nr) { return MAIN + ROWS + LO1 + (nr > 1 ? DQS : 0); }
 };
 
 // First token of token t's sequence (clamped like the forward's).
@@ -85,7 +86,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_core_kernel(BwdParams p, DqGeo 
   extern __shared__ __attribute__((aligned(256))) char lds[];
   bf16* const qs = (bf16*)(lds + L::MAIN);                 // [U][DK]
   bf16* const gs = qs + U * DK;                            // [U][DV]
-  float* const dqs = (float*)(lds + L::MAIN + L::ROWS);    // [U][32 KBN]
+  int* const lo1s = (int*)(lds + L::MAIN + L::ROWS);       // [U]
+  float* const dqs = (float*)(lds + L::MAIN + L::ROWS + L::LO1);  // [U][32 KBN]
 
   const int tid = tid_x(), lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -98,7 +100,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_core_kernel(BwdParams p, DqGeo 
   const int tq1 = min(last, (u0 + U - 1) / G);
   const int64_t kvg_k = (int64_t)g * p.k_sh, kvg_v = (int64_t)g * p.v_sh;
 
-  // the units' q and dout rows, for the partial sums
+  // the units' q and dout rows, for the partial sums, and their first short keys
+  if (tid < U) {
+    const int t = min((u0 + tid) / G, last);
+    lo1s[tid] = max(seq_start_of(p, t), t - p.ws + 1);
+  }
   for (int i = tid; i < U * (DK + DV) / 8; i += 256) {
     const int u = i / ((DK + DV) / 8), s = i % ((DK + DV) / 8);
     const int t = min((u0 + u) / G, last), h = g * G + (u0 + u) % G;
@@ -154,7 +160,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_core_kernel(BwdParams p, DqGeo 
   };
   auto dma_chunk = [&](int ch) {
     const int k0 = lo + 32 * ch;
-    if (k0 + 31 > last) offsets(last - k0);  // (the walk's last chunk)
+    // (the walk's last chunk: rows past its last query repeat that query's key,
+    // so that masked keys bring in no value that no unit sees)
+    if (k0 + 31 > tq1) offsets(tq1 - k0);
     char* const buf = lds + (ch & 1) * TAB;
     const char* kp = (const char*)uniform_ptr((const bf16*)p.k2 + (int64_t)k0 * p.k_st + kvg_k);
     const char* vp = (const char*)uniform_ptr((const bf16*)p.v2 + (int64_t)k0 * p.v_st + kvg_v);
@@ -272,10 +280,12 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_core_kernel(BwdParams p, DqGeo 
         const int t = (u0 + u) / G, h = g * G + (u0 + u) % G;
         if (t > last) continue;
         floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-        const int j0 = t - 32 * r - (R - 1);
+        // (dA is 0 in rows before the window: they take its first key, which is
+        // as finite as the window, not one the query does not see)
+        const int j0 = t - 32 * r - (R - 1), lo1 = lo1s[u];
 #pragma unroll 8
         for (int i = 0; i < R; ++i) {
-          const bf16x4 y = *(const bf16x4*)((const bf16*)p.k1 + (int64_t)max(j0 + i, 0) * p.k_st + kvg_k + col);
+          const bf16x4 y = *(const bf16x4*)((const bf16*)p.k1 + (int64_t)max(j0 + i, lo1) * p.k_st + kvg_k + col);
           const int row = u % PK * R + i;
           const floatx4 x = *(const floatx4*)(slab + (u / PK * 32 + row) * CS + 4 * (d4 ^ (row & 15)));
 #pragma unroll

@@ -37,3 +37,25 @@ def test_dq_block_edges(cuda, n, hq, hk, d, dv, ws, wl):
     for name, a, a2, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), *runs):
         assert torch.isfinite(a).all() and torch.equal(a, a2), name
         assert (a - b).abs().max().item() <= 2e-2 * max(b.abs().max().item(), 1.0), name
+
+
+@pytest.mark.parametrize("hq,hk,d,dv,ws", [(4, 1, 512, 256, 32), (8, 1, 512, 256, 16), (16, 1, 128, 128, 16),
+                                           (32, 2, 64, 64, 9)])
+def test_values_that_no_query_of_the_block_sees(cuda, hq, hk, d, dv, ws):
+    """Short rows of the sequence before (k1, v1 infinite) and keys of later
+    tokens (k2 NaN): the other queries' gradients are those of finite tensors,
+    bit for bit.  One query per workgroup here; dk1 / dv1 also gather the 31
+    queries after a key."""
+    from helpers import backward_grads
+    n, lo, hi = 140, 40, 120
+    x = [t[0] for t in rand_inputs(1, n, hq, hk, d, dv, seed=ws, device=cuda)]
+    dout = torch.randn(n, hq, dv, generator=torch.Generator().manual_seed(n)).to(x[0].dtype).to(cuda)
+    cu = torch.tensor([0, lo, n], dtype=torch.int32, device=cuda)
+    want = backward_grads(x, dout, cu, ws, 300)
+    q, k1, k2, v1, v2 = (t.clone() for t in x)
+    k1[lo - 10:lo] = float("inf")
+    v1[lo - 10:lo] = float("inf")
+    k2[hi:] = float("nan")
+    got = backward_grads((q, k1, k2, v1, v2), dout, cu, ws, 300)
+    for name, i, end in (("dq", 0, hi), ("dk1", 1, hi - 31), ("dv1", 3, hi - 31)):
+        assert torch.isfinite(want[i]).all() and torch.equal(got[i][lo:end], want[i][lo:end]), name
