@@ -293,14 +293,19 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
   } fm;
   auto form_row = [&](uint32_t block, uint32_t segs) { return 8u * (uint32_t)wid + (block * 64u + fm.lane) / segs; };
   const int fsub = PK == 1 ? 0 : 8 * wid / R;  // the unit of this wave's rows (uniform)
+  // (rows before the unit's short window, which the scores mask, take its first
+  // key: as finite as the window, where a row that the query does not see, of
+  // another sequence too, need not be)
+  int fs0[PK];  // sequence starts of the units of the step being formed
   auto form_src = [&](int st, Unit u, uint32_t row) -> const char* {
     Unit v = u;
+    int s0v = fs0[0];
 #pragma unroll
     for (int s = 1; s < PK; ++s) {
       const Unit y = advance(v);
-      if (s <= fsub) v = y;
+      if (s <= fsub) v = y, s0v = fs0[s];
     }
-    const int j = max(v.t - 32 * v.r - (R - 1) + (int)(row % R), 0);
+    const int j = max(v.t - 32 * v.r - (R - 1) + (int)(row % R), max(s0v, v.t - p.ws + 1));
     // rows of the step's own queries are still in the stage: the unit whose
     // query is j (units ascend in (t, h))
     const int st_u = PK == 1 ? 0 : min(max((j - u.t) * G - u.h, 0), PK - 1);
@@ -377,9 +382,31 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(nx));
     scal[lane] = nx;
   };
+  auto form_starts = [&](Unit u) {  // of the units of the step from u on (ascending calls)
+#pragma unroll
+    for (int s = 0; s < PK; ++s, u = advance(u)) {
+      const int t = min(u.t, tlast);
+      if (t >= snext) {  // crossed into another sequence (uniform, rare)
+        if (p.cu == nullptr) {
+          s0 = (t / p.seqlen) * p.seqlen;
+          snext = s0 + p.seqlen;
+        } else {
+          while (seq + 1 < p.num_seqs && p.cu[seq + 1] <= t) ++seq;
+          const int c = p.cu[seq];
+          s0 = min(max(c, 0), t);
+          // well formed (cu[seq] <= t): the start holds up to the next boundary
+          snext = c > t ? t + 1 : (seq + 1 < p.num_seqs ? p.cu[seq + 1] : 0x7fffffff);
+        }
+        s0 = __builtin_amdgcn_readfirstlane(s0);
+        snext = __builtin_amdgcn_readfirstlane(snext);
+      }
+      fs0[s] = s0;
+    }
+  };
   load_block(0);
   store_block();
   if (nunits > 64) load_block(1);
+  form_starts(cur);
   to_ring(0, cur);
   form_read(0, cur);
   static_for<0, UA + UB>([&](auto k) {
@@ -404,6 +431,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
     block_barrier();  // tiles of st formed, ring rows up to its queries copied, rows of st+1 staged, the other buffer free
     const Unit nx2 = after(nx1);
     dma_step(st + 2);
+    int cs0[PK];
+#pragma unroll
+    for (int s = 0; s < PK; ++s) cs0[s] = fs0[s];
+    form_starts(nx1);
 
     float lse2[PK], dpm[PK], dsm[PK];
     int ut[PK], lo2[PK], ilo[PK];
@@ -412,21 +443,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
 #pragma unroll
     for (int s = 0; s < PK; ++s, u = advance(u)) {
       ut[s] = u.t;
-      const int t = min(u.t, tlast);
-      if (t >= snext) {  // crossed into another sequence (uniform, rare)
-        if (p.cu == nullptr) {
-          s0 = (t / p.seqlen) * p.seqlen;
-          snext = s0 + p.seqlen;
-        } else {
-          while (seq + 1 < p.num_seqs && p.cu[seq + 1] <= t) ++seq;
-          const int c = p.cu[seq];
-          s0 = min(max(c, 0), t);
-          // well formed (cu[seq] <= t): the start holds up to the next boundary
-          snext = c > t ? t + 1 : (seq + 1 < p.num_seqs ? p.cu[seq + 1] : 0x7fffffff);
-        }
-        s0 = __builtin_amdgcn_readfirstlane(s0);
-        snext = __builtin_amdgcn_readfirstlane(snext);
-      }
+      const int t = min(u.t, tlast), s0 = cs0[s];
       const floatx4 sv4 = lds_read_now(scal + sl + s);
       const bool single = t == s0 || (p.ws == 1 && p.wl == 1);
       lse2[s] = uniform_f(sv4[0] * kLog2e);

@@ -45,3 +45,25 @@ def test_dkv2_step_edges(cuda, n, hq, hk, d, ws, wl, dtype):
     for name, a, a2, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), *runs):
         assert torch.isfinite(a).all() and torch.equal(a, a2), name
         assert (a - b).abs().max().item() <= tol * max(b.abs().max().item(), 1.0), name
+
+
+@pytest.mark.parametrize("hq,hk,d,dv,ws,dtype", [
+    (2, 2, 128, 128, 16, "bf16"), (6, 3, 64, 64, 8, "bf16"), (4, 2, 128, 64, 32, "bf16"), (2, 1, 64, 64, 100, "bf16"),
+    (3, 1, 256, 256, 64, "bf16"), (4, 1, 512, 256, 32, "bf16"), (4, 1, 512, 256, 5, "bf16"),
+    (4, 2, 128, 128, 32, "f32"), (2, 1, 64, 64, 7, "f32")])
+def test_short_rows_of_the_sequence_before(cuda, hq, hk, d, dv, ws, dtype):
+    """k1 and v1 rows that stand before a sequence's first token, infinite here,
+    bring nothing into its dk2 and dv2 (a key block starts at the boundary)."""
+    from helpers import backward_grads
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    lo, n = 256, 330
+    x = [t[0] for t in rand_inputs(1, n, hq, hk, d, dv, seed=ws, dtype=dt, device=cuda)]
+    dout = torch.randn(n, hq, dv, generator=torch.Generator().manual_seed(n)).to(dt).to(cuda)
+    cu = torch.tensor([0, lo, n], dtype=torch.int32, device=cuda)
+    want = backward_grads(x, dout, cu, ws, 300)
+    q, k1, k2, v1, v2 = (t.clone() for t in x)
+    k1[lo - 5:lo] = float("inf")
+    v1[lo - 9:lo] = float("inf")
+    got = backward_grads((q, k1, k2, v1, v2), dout, cu, ws, 300)
+    for name, i in (("dk2", 2), ("dv2", 4)):
+        assert torch.isfinite(want[i]).all() and torch.equal(got[i][lo:], want[i][lo:]), name
