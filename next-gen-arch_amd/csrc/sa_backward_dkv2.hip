@@ -496,26 +496,39 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
     ad.advance((st & 1) ? -TAB : TAB);  // the other buffer
     ++st;
   };
-  // Set c is reached by the steps of one range [a_c, e_c): from the query kc
-  // that is its first key to the last whose long window, cut at its sequence
-  // start, holds its last.  Two sets: the steps before set 1's range or after
-  // set 0's run one set's products (in a step that reaches neither they come
-  // out as zero), one loop each -- a choice per step would copy accumulators
-  // or branch at every product.  Every wave takes nsteps steps (barriers).
+  // Set c of a wave is reached by the steps of one range [a_c, e_c): from the
+  // query kc that is its first key to the last whose long window, cut at its
+  // sequence start, holds its last.  The steps outside a set's range leave its
+  // products out -- they would come out as zero, or NaN for values that its keys do
+  // not depend on --, one loop per choice of sets: a choice per step would copy
+  // accumulators or branch at every product.  Every wave takes nsteps steps
+  // (barriers).
+  const int64_t upt = (int64_t)G * nr;
+  auto range = [&](int c, int& a, int& e) {
+    const int kc = k0 + 128 * c + 32 * wid, kl = min(kc + 31, last);
+    if (kc > last) {  // no key: never reached
+      a = e = nsteps;
+      return;
+    }
+    const int tend = min(seq_end(kl) - 1, kl + p.wl - 1);
+    a = __builtin_amdgcn_readfirstlane((int)max((int64_t)0, min((int64_t)nsteps, (kc - tfirst) * upt / PK)));
+    e = __builtin_amdgcn_readfirstlane(
+        (int)max((int64_t)0, min((int64_t)nsteps, ((tend + 1 - tfirst) * upt + PK - 1) / PK)));
+  };
+  int a0, e0;
+  range(0, a0, e0);
+  while (st < a0) step(std::integral_constant<int, 0>{});
   if constexpr (SETS == 2) {
-    const int kc0 = k0 + 32 * wid, kc1 = kc0 + 128;
-    const int kl0 = min(kc0 + 31, last);
-    const int tend0 = min(seq_end(kl0) - 1, kl0 + p.wl - 1);  // set 0's last query
-    const int64_t upt = (int64_t)G * nr;
-    const int a1 = (int)max((int64_t)0, min((int64_t)nsteps, (kc1 - tfirst) * upt / PK));
-    const int e0 = (int)max((int64_t)0, min((int64_t)nsteps, ((tend0 + 1 - tfirst) * upt + PK - 1) / PK));
-    const int na = __builtin_amdgcn_readfirstlane(min(a1, e0)), nb = __builtin_amdgcn_readfirstlane(max(na, e0));
-    while (st < na) step(std::integral_constant<int, 1>{});
-    while (st < nb) step(std::integral_constant<int, 3>{});
-    while (st < nsteps) step(std::integral_constant<int, 2>{});
+    int a1, e1;
+    range(1, a1, e1);
+    while (st < min(a1, e0)) step(std::integral_constant<int, 1>{});
+    while (st < e0) step(std::integral_constant<int, 3>{});
+    while (st < a1) step(std::integral_constant<int, 0>{});
+    while (st < e1) step(std::integral_constant<int, 2>{});
   } else {
-    while (st < nsteps) step(std::integral_constant<int, 1>{});
+    while (st < e0) step(std::integral_constant<int, 1>{});
   }
+  while (st < nsteps) step(std::integral_constant<int, 0>{});
   write_out();
 }
 

@@ -212,12 +212,16 @@ struct BwdCore {
       return __builtin_bit_cast(bf16x8, u32x4{f.a[0], f.a[1], f.b[0], f.b[1]});
     }
   }
-  // One step for the sets in ACT (a bit mask).  sinit(c, e): start value of score
+  // One step for the sets in ACT (a bit mask; 0: the caller's work only).  sinit(c, e): start value of score
   // register e of set c (0, or the value that masks it) when `masked`.  prob(c, e, s):
   // the probability of register e of set c; grad(c, e, p, dp): its dS.
   // fill(item): the caller's work beside item 0 .. T4-1 of phase 4.
   template <int ACT, typename SI, typename PF, typename GF, typename FF>
   __device__ __forceinline__ void step(const Addr& ad, bool masked, SI&& sinit, PF&& prob, GF&& grad, FF&& fill) {
+    if constexpr (ACT == 0) {  // the caller's work only
+      static_for<0, T4>([&](auto i) { fill(i); });
+      return;
+    }
     floatx16 s[SETS], dp[SETS];
     uint32_t pk[SETS][8], pl[F32 ? SETS : 1][8];
     Frag fh[NT], fl[F32 ? NT : 1];

@@ -67,3 +67,26 @@ def test_short_rows_of_the_sequence_before(cuda, hq, hk, d, dv, ws, dtype):
     got = backward_grads((q, k1, k2, v1, v2), dout, cu, ws, 300)
     for name, i in (("dk2", 2), ("dv2", 4)):
         assert torch.isfinite(want[i]).all() and torch.equal(got[i][lo:], want[i][lo:]), name
+
+
+@pytest.mark.parametrize("hq,hk,d,dv,ws,dtype", [
+    (2, 1, 128, 128, 16, "bf16"), (4, 1, 64, 64, 8, "bf16"), (2, 2, 128, 128, 32, "bf16"), (2, 1, 256, 256, 40, "bf16"),
+    (4, 1, 512, 256, 32, "bf16"), (4, 2, 128, 128, 32, "f32"), (8, 2, 64, 64, 5, "f32")])
+def test_queries_that_do_not_reach_a_wave(cuda, hq, hk, d, dv, ws, dtype):
+    """Non-finite queries reach the 32-key groups that their long windows overlap,
+    not the rest of a workgroup's keys: a sequence before (k1 infinite) and later
+    tokens (q NaN) in the same key blocks."""
+    from helpers import backward_grads
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    lo, hi, n, wl = 96, 300, 420, 44
+    x = [t[0] for t in rand_inputs(1, n, hq, hk, d, dv, seed=ws, dtype=dt, device=cuda)]
+    dout = torch.randn(n, hq, dv, generator=torch.Generator().manual_seed(n)).to(dt).to(cuda)
+    cu = torch.tensor([0, lo, n], dtype=torch.int32, device=cuda)
+    want = backward_grads(x, dout, cu, ws, wl)
+    q, k1, k2, v1, v2 = (t.clone() for t in x)
+    k1[lo - 40:lo] = float("inf")
+    q[hi:] = float("nan")
+    got = backward_grads((q, k1, k2, v1, v2), dout, cu, ws, wl)
+    end = (hi - wl + 1) // 32 * 32
+    for name, i in (("dk2", 2), ("dv2", 4)):
+        assert torch.isfinite(want[i]).all() and torch.equal(got[i][lo:end], want[i][lo:end]), name
