@@ -154,13 +154,14 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_f32_kernel(PagedF
       s[e] = kr < klo || kr > khi ? -INFINITY : s[e] * p.sl2;
       cmax = fmaxf(cmax, s[e]);
     }
-    // (a chunk of the walk holds a valid key: the maximum is finite)
-    const float mn = fmaxf(m, pair_max(cmax)), alpha = fast_exp2(m - mn);
+    // A row whose scores so far are all -inf (they overflowed: a chunk of the walk
+    // holds a valid key) keeps sums of 0: its exponents are taken against 0.
+    const float mn = fmaxf(m, pair_max(cmax)), ref = mn == -INFINITY ? 0.f : mn, alpha = fast_exp2(m - ref);
     m = mn;
     float zs = 0.f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      s[e] = fast_exp2(s[e] - mn);
+      s[e] = fast_exp2(s[e] - ref);
       zs += s[e];
     }
     z = z * alpha + zs;

@@ -95,3 +95,30 @@ def test_rows_without_tables_match_tables(cuda, dtype, kernel, dim, n1, n2, lowe
     want = _paged_launch(q, short, long, table1, table2, torch.arange(b, device=cuda, dtype=torch.int32),
                          torch.full((b,), n - 1, device=cuda, dtype=torch.int32), n1, n, 1.0, None, False, kernel)
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("ws,wl", [(16, 200), (16, 40), (32, 200)])
+def test_scores_of_minus_infinity(cuda, ws, wl):
+    """A short key whose scores overflow to -inf over the first chunks of the
+    window, and one over all of it, weigh nothing there, as on the portable
+    kernel (whose running maximum is one for all rows); the other rows, and the
+    first one's later keys, decide the output."""
+    from archlab_amd.architectures.simplicial_paged import simplicial_paged_attention
+    n, hk, hq, dim = 230, 2, 4, 64
+    (short, long), table, _ = paged_batch([n], hk, dim, n + 2, torch.float32, seed=9, device=cuda)
+    block = table[0, 0].item()
+    q = torch.ones(1, hq, dim, device=cuda) / dim
+    seq, pos = torch.zeros(1, dtype=torch.int32, device=cuda), torch.full((1,), n - 1, dtype=torch.int32, device=cuda)
+    short[0, block, :n] = 1.0
+    short[0, block, n - 3] = 1e30    # -inf over keys of -1e30, 0 over keys of 0
+    short[0, block, n - 5] = 3e38    # -inf over every negative key
+    long[0, block, :n - 20] = -1e30
+    long[0, block, n - 20:n] = -2.0
+    long[0, block, n - 10] = 0.0
+    kw = dict(short_window=ws, long_window=wl, scale=1.0, return_lse=True)
+    for splits in (None, 1, 2):
+        out, lse = simplicial_paged_attention(q, short, long, table, seq, pos, splits=splits, **kw)
+        want, lse_ref = simplicial_paged_attention(q, short, long, table, seq, pos, kernel="generic", **kw)
+        assert torch.isfinite(want).all() and torch.isfinite(lse_ref).all()
+        torch.testing.assert_close(out, want, rtol=2e-5, atol=2e-5)
+        torch.testing.assert_close(lse, lse_ref, rtol=2e-5, atol=2e-5)
