@@ -230,7 +230,10 @@ int sa_prefill_bwd(const sa_prefill_bwd_args* args, void* workspace, size_t work
 size_t sa_paged_workspace_bytes(const sa_paged_args* args);
 
 /* Paged forward for any mix of prefill and decode tokens; workspace must hold
- * sa_paged_workspace_bytes(args) bytes (256-byte aligned). */
+ * sa_paged_workspace_bytes(args) bytes (256-byte aligned).  (fp32 queries over
+ * caches that are not both bf16 run without it too, where it is missing, too
+ * small or not aligned: in one split, on the portable kernel for short windows
+ * past 32.) */
 int sa_paged_fwd(const sa_paged_args* args, void* workspace, size_t workspace_bytes,
                  sa_stream_t stream);
 
@@ -242,7 +245,10 @@ int sa_paged_fwd(const sa_paged_args* args, void* workspace, size_t workspace_by
  * until the process ends; arguments whose partials need more (see
  * sa_paged_workspace_bytes) fail with SA_ERR_INVALID.  The call allocates
  * nothing.  Calls that overlap on one GPU share that array and race: order
- * them on one stream (or otherwise serialise them). */
+ * them on one stream (or otherwise serialise them).
+ * fp32 queries over caches that are not both bf16 use no partials here, and the
+ * array neither: one split whatever args->splits and sa_paged_splits say, or the
+ * portable kernel for short windows past 32. */
 int sa_paged_fwd_noalloc(const sa_paged_args* args, sa_stream_t stream);
 
 /* Splits the paged launch would use for these arguments (after auto-selection). */
@@ -251,9 +257,7 @@ int sa_paged_splits(const sa_paged_args* args);
 /* Name of the kernel family a call with these arguments runs: "mfma" (bf16
  * matrix-core path) or "generic" (portable path, fp32 and other shapes);
  * NULL if the arguments are invalid.  (Paged "generic" includes the fp32
- * matrix kernel of fp32 queries over caches that are not both bf16; it merges
- * split partials in sa_paged_workspace_bytes() of workspace, and does without
- * splits where the caller brings none.) */
+ * matrix kernel of fp32 queries over caches that are not both bf16.) */
 const char* sa_prefill_kernel(const sa_prefill_args* args);
 const char* sa_paged_kernel(const sa_paged_args* args);
 

@@ -284,7 +284,12 @@ int sa_paged_fwd(const sa_paged_args* a, void* workspace, size_t workspace_bytes
   if (rc != SA_OK) return rc;
   if (a->tokens == 0) return SA_OK;
   sa_paged_args c = sa::clip_paged(a);
-  if (workspace_bytes == 0 && sa::paged_f32_route(&c)) sa::paged_without_partials(&c);
+  // fp32 calls ran on the portable kernel, which takes any workspace: one that
+  // does not hold the partials is no error
+  if (sa::paged_f32_route(&c) &&
+      (!workspace || ((uintptr_t)workspace & 255) ||
+       workspace_bytes < sa::paged_workspace_bytes(&c, sa::paged_choose_splits(&c))))
+    sa::paged_without_partials(&c);
   const int splits = sa::paged_choose_splits(&c);
   const size_t need = sa::paged_workspace_bytes(&c, splits);
   if (workspace_bytes < need) return sa::fail(SA_ERR_INVALID, "workspace too small");

@@ -311,6 +311,24 @@ def test_paged_plan_bounds_a_global_short_window():
     assert ws <= splits * 16 * 4 * 32 * 130 * 4 + 3 * 256, ws
 
 
+@pytest.mark.parametrize("short_window", [16, 40])
+def test_fp32_paged_calls_take_any_workspace(short_window):
+    """An fp32 query over fp32 caches needed no workspace on the portable kernel:
+    a missing, small or unaligned one is no argument error now that splits would
+    use one (without a GPU such a call gets as far as its launch)."""
+    from archlab_amd import _native
+    if torch.cuda.is_available():
+        pytest.skip("launches on made-up addresses are for machines without a GPU")
+    lib = _native.load()
+    args = _c5_plan_args(short_window, 4096, tokens=4, table_width=64)
+    args.q_dtype = args.cache_dtype = args.long_cache_dtype = _native.SA_DTYPE_F32
+    need = lib.sa_paged_workspace_bytes(ctypes.byref(args))
+    assert need > 4096
+    base = 1 << 20
+    for workspace, nbytes in ((None, 0), (base, 0), (base, 4096), (None, need), (base + 16, need), (base, need - 1)):
+        assert lib.sa_paged_fwd(ctypes.byref(args), workspace, nbytes, None) == _native.SA_ERR_HIP, (workspace, nbytes)
+
+
 def test_window_lengths_beyond_int32_saturate():
     from archlab_amd import _native
     assert _native.window(2 ** 32 + 100) == 2 ** 31 - 1
