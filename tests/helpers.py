@@ -59,6 +59,19 @@ def assert_lse_close(actual, expected, dtype, rtol=None):
     return rel
 
 
+def assert_grads_close(actual, expected, rel_max, rel_norm):
+    """dq, dk1, dk2, dv1, dv2 each within rel_max of its own largest value and
+    rel_norm of its norm (no absolute floor: dk1 and dk2 are small)."""
+    for name, a, e in zip(("dq", "dk1", "dk2", "dv1", "dv2"), actual, expected):
+        a, e = a.float(), e.float()
+        assert torch.isfinite(a).all(), f"{name}: non-finite"
+        diff, norm = (a - e).abs().max().item(), (a - e).norm().item()
+        print(f"{name}: max {diff / max(e.abs().max().item(), 1e-30):.1e}, "
+              f"norm {norm / max(e.norm().item(), 1e-30):.1e}", flush=True)
+        assert diff <= rel_max * e.abs().max().item(), f"{name}: {diff:.2e}"
+        assert norm <= rel_norm * e.norm().item(), f"{name}: {norm:.2e} of {e.norm().item():.2e}"
+
+
 def paged_batch(lengths, kv_heads, dim, block_size, dtype, hnd=False, seed=0, device="cuda"):
     """Contiguous per-sequence K/V plus the same rows scattered into shuffled pages.
 

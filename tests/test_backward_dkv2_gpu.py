@@ -2,14 +2,18 @@
 around the 8- and 16-key steps (two or four units per 32-row step), groups that
 leave the last step partly filled, key blocks of 256 and 128 with a remainder,
 row groups past the first, and sequences that end inside a key block.  Checked
-with all five gradients against the portable kernels (same rounding points,
-another order of the fp32 sums: 2e-2 of the largest gradient in bf16, 1e-4 in
-fp32) and for repeatability."""
+with all five gradients against the portable kernels and for repeatability.
+
+Same rounding points, another order of the fp32 sums: in bf16 the forward's O and
+a few P and dS round the other way (2^-8 of a term), and the results once more, so
+that a gradient moves by about 2e-3 of its norm and at most some 2^-7 of its
+largest value; a dropped unit, row group or piece of one of these shapes is a
+percent or more.  fp32: hi/lo terms, 2^-16."""
 
 import pytest
 import torch
 
-from helpers import rand_inputs
+from helpers import assert_grads_close, rand_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -39,12 +43,10 @@ def test_dkv2_step_edges(cuda, n, hq, hk, d, ws, wl, dtype):
     runs = []
     for kernel in ("auto", "auto", "generic"):
         xd = [t.clone().requires_grad_(True) for t in x]
-        simplicial_varlen_attention(*xd, cu, ws, wl, kernel=kernel).backward(dout)
+        simplicial_varlen_attention(*xd, cu, ws, wl, scale=1.0, kernel=kernel).backward(dout)
         runs.append([t.grad.float() for t in xd])
-    tol = 2e-2 if dtype == "bf16" else 1e-4
-    for name, a, a2, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), *runs):
-        assert torch.isfinite(a).all() and torch.equal(a, a2), name
-        assert (a - b).abs().max().item() <= tol * max(b.abs().max().item(), 1.0), name
+    assert all(torch.equal(a, a2) for a, a2 in zip(*runs[:2]))
+    assert_grads_close(runs[0], runs[2], *((2e-2, 5e-3) if dtype == "bf16" else (1e-4, 1e-4)))
 
 
 @pytest.mark.parametrize("hq,hk,d,dv,ws,dtype", [

@@ -1,13 +1,15 @@
 """dq / dk1 / dv1 pass at the edges of its workgroups: groups that divide a
 workgroup's units, are divided by them or neither, last units past the tokens,
 short windows at the 16-key units, and sequences that end inside a workgroup.
-All five gradients against the portable kernels (same rounding points, another
-order of the fp32 sums: 2e-2 of the largest gradient) and for repeatability."""
+All five gradients against the portable kernels and for repeatability (same
+rounding points, another order of the fp32 sums: some terms and the results round
+the other way, about 2e-3 of a gradient's norm and at most some 2^-7 of its
+largest value)."""
 
 import pytest
 import torch
 
-from helpers import rand_inputs
+from helpers import assert_grads_close, rand_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -32,11 +34,10 @@ def test_dq_block_edges(cuda, n, hq, hk, d, dv, ws, wl):
     runs = []
     for kernel in ("auto", "auto", "generic"):
         xd = [t.clone().requires_grad_(True) for t in x]
-        simplicial_varlen_attention(*xd, cu, ws, wl, kernel=kernel).backward(dout)
+        simplicial_varlen_attention(*xd, cu, ws, wl, scale=1.0, kernel=kernel).backward(dout)
         runs.append([t.grad.float() for t in xd])
-    for name, a, a2, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), *runs):
-        assert torch.isfinite(a).all() and torch.equal(a, a2), name
-        assert (a - b).abs().max().item() <= 2e-2 * max(b.abs().max().item(), 1.0), name
+    assert all(torch.equal(a, a2) for a, a2 in zip(*runs[:2]))
+    assert_grads_close(runs[0], runs[2], 2e-2, 5e-3)
 
 
 @pytest.mark.parametrize("hq,hk,d,dv,ws", [(4, 1, 512, 256, 32), (8, 1, 512, 256, 16), (16, 1, 128, 128, 16),

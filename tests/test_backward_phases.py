@@ -64,7 +64,7 @@ def test_phases_cover_every_block_and_key(tmp_path):
 def _against_portable(cuda, n, hq, hk, d, dv, ws, wl, flags):
     import torch
     from archlab_amd import _native
-    from helpers import backward_grads, rand_inputs
+    from helpers import assert_grads_close, backward_grads, rand_inputs
     x = [t[0] for t in rand_inputs(1, n, hq, hk, d, dv, seed=n + ws, device=cuda)]
     dout = torch.randn(n, hq, dv, generator=torch.Generator().manual_seed(n)).to(x[0].dtype).to(cuda)
     cu = torch.tensor([0, n // 3, n], dtype=torch.int32, device=cuda)
@@ -72,13 +72,10 @@ def _against_portable(cuda, n, hq, hk, d, dv, ws, wl, flags):
     got = backward_grads(x, dout, cu, ws, wl, flags, scratch)
     again = backward_grads(x, dout, cu, ws, wl, flags)
     want = backward_grads(x, dout, cu, ws, wl, _native.SA_FLAG_FORCE_GENERIC)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
     # the same rounding points in another order of the fp32 sums: some P and dS
     # round the other way (2^-8 of a term), and the results once more
-    for name, a, a2, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), got, again, want):
-        a, b = a.float(), b.float()
-        assert torch.isfinite(a).all() and torch.equal(got[0], again[0]) and torch.equal(a, a2.float()), name
-        assert (a - b).norm() <= 1e-2 * b.norm(), name
-        assert (a - b).abs().max() <= 2e-2 * b.abs().max(), name
+    assert_grads_close(got, want, 2e-2, 5e-3)
     return scratch[0]
 
 
