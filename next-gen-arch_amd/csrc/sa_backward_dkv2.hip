@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv2_kernel(BwdParams p, Dkv2Geo g
     const int inrow = b - (isq ? 0 : isg ? RBK : isk ? RKV : RKV + RBK);
     dptr[k] = (const char*)(base + (int64_t)tfirst * st_t + (int64_t)(isg ? g * G : g) * st_h) + inrow;
     dhead[k] = isg ? (int)(st_h / 8) : 0;
-    dtok[k] = (int)(st_t / 8) - (isg ? (G - 1) * (int)(st_h / 8) : 0);
+    dtok[k] = (int)walk_query_step(st_t / 8, st_h / 8, isg ? G : 1);
   }
   Unit dunit{tfirst, 0, 0};
   auto dma_step = [&](int st) {  // called for st = 0, 1, 2, ..
@@ -633,6 +633,10 @@ int64_t dkv2_piece_bytes(int tokens, int hk, int d, int dv) { return (int64_t)to
 // k1 / v1 ring's LDS); fp32 inputs 32 (the other fp32 passes' bound).
 hipError_t launch_bwd_dkv2_mfma(const BwdParams& p, size_t scratch_bytes, hipStream_t stream) {
   if (!bwd_mfma_ok(p)) return hipErrorNotSupported;
+  const int per16 = p.f32 ? 4 : 8;  // elements per 16 bytes
+  if (!walk_steps_fit(p.q_st / per16, p.q_sh / per16, p.group) || !walk_steps_fit(p.do_st / per16, p.do_sh / per16, p.group) ||
+      !walk_steps_fit(p.k_st / per16, 0, 1) || !walk_steps_fit(p.v_st / per16, 0, 1))
+    return hipErrorNotSupported;
   if (p.f32) {
     if (p.ws > 32) return hipErrorNotSupported;
     if (p.d == 128) return launch_dkv2_pk<128, 128, 1, true>(p, scratch_bytes, stream);

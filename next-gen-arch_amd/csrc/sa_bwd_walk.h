@@ -28,6 +28,17 @@ constexpr bool walk_moves(WalkUnit u, WalkUnit y, int i, int n, int pk) {
 }
 
 
+// Pointer steps between staged rows, in 16-byte units (strides in the same): the
+// next head's row, and from the last head of a query to the first of the next.
+// The kernel holds them in 32 bits.
+constexpr long long walk_query_step(long long stride_t, long long stride_h, int group) {
+  return stride_t - (group - 1) * stride_h;
+}
+constexpr bool walk_steps_fit(long long stride_t, long long stride_h, int group) {
+  const long long q = walk_query_step(stride_t, stride_h, group), lim = 0x7fffffffLL;
+  return stride_h >= -lim && stride_h <= lim && q >= -lim && q <= lim;
+}
+
 // dq / dk1 / dv1 pass: blocks of U consecutive units (t, h), whose partials may
 // take more space than there is (room for `cap` blocks).  It then runs in
 // phases, blocks [b0, b0 + nb) each, followed by the sums of the keys [j0, j1)

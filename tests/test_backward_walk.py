@@ -42,6 +42,16 @@ int main() {
             }
           }
       }
+  // pointer steps: head-major strides of large tensors pass 32 bits
+  for (long long tokens : {1000LL, 1LL << 20, 1LL << 24})
+    for (int group : {1, 2, 64, 128})
+      for (long long row : {8LL, 32LL})  // 16-byte units of a row
+        for (int major : {0, 1, -1}) {
+          const long long st_t = major ? row : group * row, st_h = major ? major * tokens * row : row;
+          const long long q = st_t - (group - 1) * st_h;
+          const bool fit = (int)st_h == st_h && (int)q == q;
+          if (walk_steps_fit(st_t, st_h, group) != fit || walk_query_step(st_t, st_h, group) != q) ++bad;
+        }
   printf("%ld units, %ld off\n", units, bad);
   return bad != 0;
 }
