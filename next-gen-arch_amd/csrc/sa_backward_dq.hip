@@ -3,11 +3,11 @@
 //
 // A workgroup of 4 waves owns U consecutive units (query t, head h of one KV
 // group); a wave holds SETS x 32 of their rows j as MFMA fragments, A rows
-// bf16(q_th ⊙ k1_j) and B rows bf16(dout_th ⊙ v1_j): one unit's 32-row group
-// of short keys per set or, with short windows of at most 16 (8) keys, PK = 2
-// (4) units of 16 (8) rows.  The waves walk the chunks of 32 long keys that
-// the units reach, whose K2 / V2 rows stream into LDS (double-buffered DMAs, one
-// barrier per chunk).  Per set (BwdCore, keys x rows j):
+// bf16(q_th ⊙ k1_j) and B rows bf16(dout_th ⊙ v1_j): one unit's 32 short keys
+// per set or, with short windows of at most 16, PK = 2 units of 16 rows.  The
+// waves walk the chunks of 32 long keys that the units reach, whose K2 / V2 rows
+// stream into LDS (double-buffered DMAs, one barrier per chunk).  Per set
+// (BwdCore, keys x rows j):
 //     S = K2 · A^T,  dP = V2 · B^T,  O''^T += V2^T · P,  dA^T += K2^T · dS
 // After the walk dA and O'' go through LDS, where
 //     dq_th = Σ_j dA_j ⊙ k1_j     dk1_j += Σ_th dA_j ⊙ q_th     dv1_j += Σ_th O''_j ⊙ dout_th
@@ -49,9 +49,8 @@ namespace {
 struct DqGeo {
   int nblocks;  // workgroups of the launch
   int b0, nb;   // blocks [b0, b0 + nb) of every KV head
-  int nr;       // 32-row groups of short keys (1 with PK > 1)
   int nrows;    // short-key rows of a block's partial
-  float* part;  // [hk][nb][nr][nrows][DK + DV]
+  float* part;  // [hk][nb][nrows][DK + DV]
 };
 
 template <int DK, int DV, int SETS, int PK, int KBN>
@@ -62,8 +61,7 @@ struct DqLds {
   static constexpr int MAIN = 2 * TAB > S * 32 * CS * 4 ? 2 * TAB : S * 32 * CS * 4;
   static constexpr int ROWS = U * 2 * (DK + DV);                // q and dout rows of the units
   static constexpr int LO1 = U * 4;                             // first short key of the units
-  static constexpr int DQS = U * 32 * KBN * 4;                  // dq sums over row groups
-  static constexpr size_t bytes(int nr) { return MAIN + ROWS + LO1 + (nr > 1 ? DQS : 0); }
+  static constexpr size_t BYTES = MAIN + ROWS + LO1;
 };
 
 // First token of token t's sequence (clamped like the forward's).
@@ -87,7 +85,6 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_core_kernel(BwdParams p, DqGeo 
   bf16* const qs = (bf16*)(lds + L::MAIN);                 // [U][DK]
   bf16* const gs = qs + U * DK;                            // [U][DV]
   int* const lo1s = (int*)(lds + L::MAIN + L::ROWS);       // [U]
-  float* const dqs = (float*)(lds + L::MAIN + L::ROWS + L::LO1);  // [U][32 KBN]
 
   const int tid = tid_x(), lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -176,149 +173,140 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_core_kernel(BwdParams p, DqGeo 
   const float smask = p.scale < 0.f ? INFINITY : -INFINITY;
   C core;
 
-  for (int r = 0; r < geo.nr; ++r) {
-    if (r > 0) __syncthreads();  // the epilogue's slab is read
-    offsets(31);
-    dma_chunk(0);
-    float bias[SETS], dpm[SETS], dsm[SETS];
+  offsets(31);
+  dma_chunk(0);
+  float bias[SETS], dpm[SETS], dsm[SETS];
+#pragma unroll
+  for (int c = 0; c < SETS; ++c) {
+    const int j = ut[c] - (R - 1) + n % R;
+    const bool ok = uok[c] && j >= max(us0[c], ut[c] - p.ws + 1);
+    const int jc = max(j, 0);
+    const bf16* qr = (const bf16*)p.q + (int64_t)ut[c] * p.q_st + uth[c] * p.q_sh + 8 * half;
+    const bf16* gr = (const bf16*)p.dout + (int64_t)ut[c] * p.do_st + uth[c] * p.do_sh + 8 * half;
+    const bf16* k1r = (const bf16*)p.k1 + (int64_t)jc * p.k_st + kvg_k + 8 * half;
+    const bf16* v1r = (const bf16*)p.v1 + (int64_t)jc * p.v_st + kvg_v + 8 * half;
+    auto form = [&](const bf16* a, const bf16* bb) {
+      const u32x4 x = *(const u32x4*)a, y = *(const u32x4*)bb;
+      u32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = ok ? mul_bf16_pair(x[e], y[e]) : 0u;
+      return __builtin_bit_cast(bf16x8, o);
+    };
+#pragma unroll
+    for (int t = 0; t < DK / 16; ++t) core.kx[c][t] = form(qr + 16 * t, k1r + 16 * t);
+#pragma unroll
+    for (int t = 0; t < DV / 16; ++t) core.vx[c][t] = form(gr + 16 * t, v1r + 16 * t);
+    const int64_t thq = (int64_t)ut[c] * p.hq + uth[c];
+    const float lse = p.lse[(int64_t)ut[c] * p.lse_st + uth[c]];
+    const bool single = ut[c] == us0[c] || (p.ws == 1 && p.wl == 1);
+    bias[c] = ok ? lse * kLog2e : INFINITY;  // (p = 0 in rows outside the short window)
+    dpm[c] = single ? 0.f : p.scale;
+    dsm[c] = single ? p.dl[thq] * p.scale : -p.delta[thq] * p.scale;
+  }
+  core.clear();
+  typename C::Addr ad = C::addresses(lds, lds + C::TK, 0, lane);
+  for (int ch = 0; ch < nch; ++ch) {
+    wait_vmcnt<0>();
+    block_barrier();  // chunk ch has landed, the other buffer is free
+    if (ch + 1 < nch) dma_chunk(ch + 1);
+    const int k0 = lo + 32 * ch;
+    const bool masked = k0 < lo_last || k0 + 31 > tq0;
+    auto sinit = [&](int c, int e) {
+      const int kr = k0 + 8 * (e >> 2) + (e & 3) + 4 * half;
+      return kr < ulo[c] || kr > ut[c] ? smask : 0.f;
+    };
+    auto prob = [&](int c, int, float s) { return fast_exp2(fmaf(s, sl2s, -bias[c])); };
+    auto grad = [&](int c, int, float pr, float dp) { return pr * fmaf(dp, dpm[c], dsm[c]); };
+    core.template step<(1 << SETS) - 1>(ad, masked, sinit, prob, grad, [](auto) {});
+    ad.advance((ch & 1) ? -TAB : TAB);
+  }
+  acc_settle();
+  __syncthreads();  // every wave is done with the tiles: slabs take their place
+
+  const int lf = fresh_lane(), tf = 64 * wid + lf;
+  float* const slab = (float*)lds;  // [S][32][CS], 16-byte segment s of row n at s ^ (n % 16)
+  constexpr int C4 = CS / 4, TRG = 256 / C4, NRT = (R - 1 + U + TRG - 1) / TRG;
+  const int d4 = tf % C4, rg = tf / C4;
+  // the block's partial rows of 32 x nblk columns from d0 (K: dA with q; V: O'' with dout)
+  auto partial = [&](const bf16* xs, int width, int col, int pcol) {
+    floatx4 acc[NRT];
+#pragma unroll
+    for (int i = 0; i < NRT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    int t = tq0, h = h0;
+    for (int u = 0; u < U && t <= last; ++u) {
+      const bf16x4 x4 = *(const bf16x4*)(xs + u * width + col);
+      const floatx4 x = {(float)x4[0], (float)x4[1], (float)x4[2], (float)x4[3]};
+#pragma unroll
+      for (int i = 0; i < NRT; ++i) {
+        const int nn = rg + TRG * i - (t - tq0);
+        if (nn < 0 || nn >= R) continue;
+        const int row = u % PK * R + nn;
+        acc[i] += *(const floatx4*)(slab + (u / PK * 32 + row) * CS + 4 * (d4 ^ (row & 15))) * x;
+      }
+      if (++h == G) h = 0, ++t;
+    }
+    float* const dst = geo.part + ((int64_t)g * geo.nb + (b - geo.b0)) * geo.nrows * (DK + DV) + pcol;
+#pragma unroll
+    for (int i = 0; i < NRT; ++i)
+      if (rg + TRG * i < geo.nrows) *(floatx4*)(dst + (int64_t)(rg + TRG * i) * (DK + DV)) = acc[i];
+  };
+  auto put = [&](const floatx16& a, int c, int db) {  // one 32-column block of a set into the slab
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      floatx4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = acc_get(a, 4 * q4 + e);
+      const int row = lf & 31;
+      *(floatx4*)(slab + ((wid * SETS + c) * 32 + row) * CS + 4 * ((8 * db + 2 * q4 + (lf >> 5)) ^ (row & 15))) = x;
+    }
+  };
+  static_for<0, 32 * KBN / CS>([&](auto ss) {
+    constexpr int s = decltype(ss)::value;
+    if (s > 0) __syncthreads();
 #pragma unroll
     for (int c = 0; c < SETS; ++c) {
-      const int j = ut[c] - 32 * r - (R - 1) + n % R;
-      const bool ok = uok[c] && j >= max(us0[c], ut[c] - p.ws + 1);
-      const int jc = max(j, 0);
-      const bf16* qr = (const bf16*)p.q + (int64_t)ut[c] * p.q_st + uth[c] * p.q_sh + 8 * half;
-      const bf16* gr = (const bf16*)p.dout + (int64_t)ut[c] * p.do_st + uth[c] * p.do_sh + 8 * half;
-      const bf16* k1r = (const bf16*)p.k1 + (int64_t)jc * p.k_st + kvg_k + 8 * half;
-      const bf16* v1r = (const bf16*)p.v1 + (int64_t)jc * p.v_st + kvg_v + 8 * half;
-      auto form = [&](const bf16* a, const bf16* bb) {
-        const u32x4 x = *(const u32x4*)a, y = *(const u32x4*)bb;
-        u32x4 o;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = ok ? mul_bf16_pair(x[e], y[e]) : 0u;
-        return __builtin_bit_cast(bf16x8, o);
-      };
-#pragma unroll
-      for (int t = 0; t < DK / 16; ++t) core.kx[c][t] = form(qr + 16 * t, k1r + 16 * t);
-#pragma unroll
-      for (int t = 0; t < DV / 16; ++t) core.vx[c][t] = form(gr + 16 * t, v1r + 16 * t);
-      const int64_t thq = (int64_t)ut[c] * p.hq + uth[c];
-      const float lse = p.lse[(int64_t)ut[c] * p.lse_st + uth[c]];
-      const bool single = ut[c] == us0[c] || (p.ws == 1 && p.wl == 1);
-      bias[c] = ok ? lse * kLog2e : INFINITY;  // (p = 0 in rows outside the short window)
-      dpm[c] = single ? 0.f : p.scale;
-      dsm[c] = single ? p.dl[thq] * p.scale : -p.delta[thq] * p.scale;
+      for (int i = 0; i < CS / 32; ++i) put(core.ak[c][s * (CS / 32) + i], c, i);
     }
-    core.clear();
-    typename C::Addr ad = C::addresses(lds, lds + C::TK, 0, lane);
-    for (int ch = 0; ch < nch; ++ch) {
-      wait_vmcnt<0>();
-      block_barrier();  // chunk ch has landed, the other buffer is free
-      if (ch + 1 < nch) dma_chunk(ch + 1);
-      const int k0 = lo + 32 * ch;
-      const bool masked = k0 < lo_last || k0 + 31 > tq0;
-      auto sinit = [&](int c, int e) {
-        const int kr = k0 + 8 * (e >> 2) + (e & 3) + 4 * half;
-        return kr < ulo[c] || kr > ut[c] ? smask : 0.f;
-      };
-      auto prob = [&](int c, int, float s) { return fast_exp2(fmaf(s, sl2s, -bias[c])); };
-      auto grad = [&](int c, int, float pr, float dp) { return pr * fmaf(dp, dpm[c], dsm[c]); };
-      core.template step<(1 << SETS) - 1>(ad, masked, sinit, prob, grad, [](auto) {});
-      ad.advance((ch & 1) ? -TAB : TAB);
-    }
-    acc_settle();
-    __syncthreads();  // every wave is done with the tiles: slabs take their place
-
-    const int lf = fresh_lane(), tf = 64 * wid + lf;
-    float* const slab = (float*)lds;  // [S][32][CS], 16-byte segment s of row n at s ^ (n % 16)
-    constexpr int C4 = CS / 4, TRG = 256 / C4, NRT = (R - 1 + U + TRG - 1) / TRG;
-    const int d4 = tf % C4, rg = tf / C4;
-    // the block's partial rows of 32 x nblk columns from d0 (K: dA with q; V: O'' with dout)
-    auto partial = [&](const bf16* xs, int width, int col, int pcol) {
-      floatx4 acc[NRT];
-#pragma unroll
-      for (int i = 0; i < NRT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-      int t = tq0, h = h0;
-      for (int u = 0; u < U && t <= last; ++u) {
-        const bf16x4 x4 = *(const bf16x4*)(xs + u * width + col);
-        const floatx4 x = {(float)x4[0], (float)x4[1], (float)x4[2], (float)x4[3]};
-#pragma unroll
-        for (int i = 0; i < NRT; ++i) {
-          const int nn = rg + TRG * i - (t - tq0);
-          if (nn < 0 || nn >= R) continue;
-          const int row = u % PK * R + nn;
-          acc[i] += *(const floatx4*)(slab + (u / PK * 32 + row) * CS + 4 * (d4 ^ (row & 15))) * x;
-        }
-        if (++h == G) h = 0, ++t;
-      }
-      float* const dst = geo.part + (((int64_t)g * geo.nb + (b - geo.b0)) * geo.nr + r) * geo.nrows * (DK + DV) + pcol;
-#pragma unroll
-      for (int i = 0; i < NRT; ++i)
-        if (rg + TRG * i < geo.nrows) *(floatx4*)(dst + (int64_t)(rg + TRG * i) * (DK + DV)) = acc[i];
-    };
-    auto put = [&](const floatx16& a, int c, int db) {  // one 32-column block of a set into the slab
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        floatx4 x;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = acc_get(a, 4 * q4 + e);
-        const int row = lf & 31;
-        *(floatx4*)(slab + ((wid * SETS + c) * 32 + row) * CS + 4 * ((8 * db + 2 * q4 + (lf >> 5)) ^ (row & 15))) = x;
-      }
-    };
-    static_for<0, 32 * KBN / CS>([&](auto ss) {
-      constexpr int s = decltype(ss)::value;
-      if (s > 0) __syncthreads();
-#pragma unroll
-      for (int c = 0; c < SETS; ++c) {
-#pragma unroll
-        for (int i = 0; i < CS / 32; ++i) put(core.ak[c][s * (CS / 32) + i], c, i);
-      }
-      __syncthreads();
-      const int col = 32 * KB0 + CS * s + 4 * d4;
-      partial(qs, DK, col, col);
-      for (int u = rg; u < U; u += TRG) {  // dq of one unit: its rows times k1
-        const int t = (u0 + u) / G, h = g * G + (u0 + u) % G;
-        if (t > last) continue;
-        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-        // (dA is 0 in rows before the window: they take its first key, which is
-        // as finite as the window, not one the query does not see)
-        const int j0 = t - 32 * r - (R - 1), lo1 = lo1s[u];
+    __syncthreads();
+    const int col = 32 * KB0 + CS * s + 4 * d4;
+    partial(qs, DK, col, col);
+    for (int u = rg; u < U; u += TRG) {  // dq of one unit: its rows times k1
+      const int t = (u0 + u) / G, h = g * G + (u0 + u) % G;
+      if (t > last) continue;
+      floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+      // (dA is 0 in rows before the window: they take its first key, which is
+      // as finite as the window, not one the query does not see)
+      const int j0 = t - (R - 1), lo1 = lo1s[u];
 #pragma unroll 8
-        for (int i = 0; i < R; ++i) {
-          const bf16x4 y = *(const bf16x4*)((const bf16*)p.k1 + (int64_t)max(j0 + i, lo1) * p.k_st + kvg_k + col);
-          const int row = u % PK * R + i;
-          const floatx4 x = *(const floatx4*)(slab + (u / PK * 32 + row) * CS + 4 * (d4 ^ (row & 15)));
+      for (int i = 0; i < R; ++i) {
+        const bf16x4 y = *(const bf16x4*)((const bf16*)p.k1 + (int64_t)max(j0 + i, lo1) * p.k_st + kvg_k + col);
+        const int row = u % PK * R + i;
+        const floatx4 x = *(const floatx4*)(slab + (u / PK * 32 + row) * CS + 4 * (d4 ^ (row & 15)));
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[e], (float)y[e], acc[e]);
-        }
-        float* const sum = dqs + u * 32 * KBN + CS * s + 4 * d4;  // (this thread's alone)
-        if (r > 0) acc += *(const floatx4*)sum;
-        if (r + 1 < geo.nr) {
-          *(floatx4*)sum = acc;
-        } else {
-          bf16x4 o;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = (bf16)acc[e];
-          *(bf16x4*)((bf16*)p.dq + (int64_t)t * p.dq_st + (int64_t)h * p.dq_sh + col) = o;
-        }
+        for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[e], (float)y[e], acc[e]);
       }
-    });
-    static_for<0, 32 * VBN / CS>([&](auto ss) {
-      constexpr int s = decltype(ss)::value;
-      __syncthreads();
+      bf16x4 o;
 #pragma unroll
-      for (int c = 0; c < SETS; ++c) {
+      for (int e = 0; e < 4; ++e) o[e] = (bf16)acc[e];
+      *(bf16x4*)((bf16*)p.dq + (int64_t)t * p.dq_st + (int64_t)h * p.dq_sh + col) = o;
+    }
+  });
+  static_for<0, 32 * VBN / CS>([&](auto ss) {
+    constexpr int s = decltype(ss)::value;
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < CS / 32; ++i) put(core.av[c][s * (CS / 32) + i], c, i);
-      }
-      __syncthreads();
-      partial(gs, DV, CS * s + 4 * d4, DK + CS * s + 4 * d4);
-    });
-  }
+    for (int c = 0; c < SETS; ++c) {
+#pragma unroll
+      for (int i = 0; i < CS / 32; ++i) put(core.av[c][s * (CS / 32) + i], c, i);
+    }
+    __syncthreads();
+    partial(gs, DV, CS * s + 4 * d4, DK + CS * s + 4 * d4);
+  });
 }
 
-// dk1 and dv1 of the keys [j0, j1): their blocks' partials in (row group,
-// block) order; 4 values per thread.
+// dk1 and dv1 of the keys [j0, j1): their blocks' partials in block order; 4
+// values per thread.
 __global__ __launch_bounds__(256) void bwd_dk1_dv1_sum_kernel(BwdParams p, DqGeo geo, int U, int R, int j0, int j1) {
   const int w = p.d + p.dv;
   const int64_t i = (int64_t)bid_x() * 256 + tid_x();
@@ -328,15 +316,11 @@ __global__ __launch_bounds__(256) void bwd_dk1_dv1_sum_kernel(BwdParams p, DqGeo
   const int g = (int)(jg % p.hk), j = j0 + (int)(jg / p.hk);
   const int G = p.group;
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int r = 0; r < geo.nr; ++r) {
-    const int tlo = j + 32 * r, thi = min(tlo + R - 1, p.tokens - 1);
-    if (tlo >= p.tokens) break;
-    const int blo = (int)((int64_t)tlo * G / U), bhi = (int)(((int64_t)thi * G + G - 1) / U);
-    for (int b = blo; b <= bhi; ++b) {
-      const int tq0 = (int)((int64_t)b * U / G);
-      const int row = tlo - tq0 + R - 1;
-      acc += *(const floatx4*)(geo.part + ((((int64_t)g * geo.nb + (b - geo.b0)) * geo.nr + r) * geo.nrows + row) * w + c);
-    }
+  const int thi = min(j + R - 1, p.tokens - 1);
+  const int blo = (int)((int64_t)j * G / U), bhi = (int)(((int64_t)thi * G + G - 1) / U);
+  for (int b = blo; b <= bhi; ++b) {
+    const int row = j - (int)((int64_t)b * U / G) + R - 1;
+    acc += *(const floatx4*)(geo.part + (((int64_t)g * geo.nb + (b - geo.b0)) * geo.nrows + row) * w + c);
   }
   const bool isk = c < p.d;
   bf16x4 o;
@@ -349,7 +333,7 @@ __global__ __launch_bounds__(256) void bwd_dk1_dv1_sum_kernel(BwdParams p, DqGeo
 
 template <int DK, int DV, int SETS, int PK, int KB0, int KBN, int VBN>
 hipError_t launch_dq_slice(const BwdParams& p, const DqGeo& geo, hipStream_t stream) {
-  const size_t lds = DqLds<DK, DV, SETS, PK, KBN>::bytes(geo.nr);
+  constexpr size_t lds = DqLds<DK, DV, SETS, PK, KBN>::BYTES;
   auto kern = bwd_dq_core_kernel<DK, DV, SETS, PK, KB0, KBN, VBN>;
   hipError_t e = set_lds_limit((const void*)kern, lds);
   if (e != hipSuccess) return e;
@@ -363,13 +347,13 @@ inline int block_queries(int U, int G) { return U % G == 0 ? U / G : G % U == 0 
 template <int DK, int DV, int SETS, int PK>
 hipError_t launch_dq_t(const BwdParams& p, size_t scratch_bytes, hipStream_t stream) {
   constexpr int U = 4 * SETS * PK, R = 32 / PK;
+  if (p.ws > R) return hipErrorNotSupported;
   DqGeo geo{};
-  geo.nr = PK > 1 ? 1 : (p.ws + 31) / 32;
   geo.nrows = R - 1 + block_queries(U, p.group);
   geo.part = p.dkv2s;
-  const int64_t bytes = (int64_t)p.hk * geo.nr * geo.nrows * (DK + DV) * sizeof(float);  // of a block of every KV head
+  const int64_t bytes = (int64_t)p.hk * geo.nrows * (DK + DV) * sizeof(float);  // of a block of every KV head
   const int64_t cap = (int64_t)(scratch_bytes / bytes);
-  const int reach = R - 1 + 32 * (geo.nr - 1);  // queries after its own that a key waits for
+  constexpr int reach = R - 1;  // queries after its own that a key waits for
   // (score width 512: the portable kernels otherwise)
   const int64_t least = DK > 256 ? 1 : device_cu_count() / 2 / p.hk + 1;
   if (!dq_phases_pay(p.tokens, p.group, U, reach, cap, least)) return hipErrorNotSupported;
