@@ -206,23 +206,33 @@ typedef struct sa_prefill_bwd_args {
  *   none with SA_FLAG_SEPARATE_DK1 in args->fwd.flags; fp32 calls also hold
  *   the dq pass's dv1 partials, the same size at value_dim (dk1 and dv1
  *   partials together up to 8 GiB, else the dv1 pass runs);
- * - for short windows of 65-128 (33-64 at head_dim 256), the fp32 dk2 and dv2
- *   sums of the first of two dk2 / dv2 launches ([tokens][heads_kv][head_dim +
+ * - for bf16 at short windows of 65-128 (33-64 at head_dim 256), room for fp32
+ *   sums of the dk2 / dv2 pass's walk pieces ([tokens][heads_kv][head_dim +
  *   value_dim]);
  * - for fp32 inputs on the matrix cores, k2 and v2 as hi/lo bf16 rows
  *   ([tokens][heads_kv][2 head_dim] each);
  * - for bf16 at head_dim 512 over value_dim 256 and short windows <= 32, the
- *   partials of dk1 and dv1 (24-25.5x the bytes of q at GQA groups of 4, up to
- *   2 GiB; none with SA_FLAG_SEPARATE_DK1, which leaves those passes to the
- *   portable kernels);
+ *   partials of dk1 and dv1 (at GQA groups of 4 24x the bytes of q, 6.4x with at
+ *   most 16 short keys; up to 2 GiB, past which the pass runs in phases; none with
+ *   SA_FLAG_SEPARATE_DK1, which leaves those passes to the portable kernels);
  * - for bf16 at widths 64 / 128 and short windows <= 64 whose (key block, KV
- *   head) work leaves CUs idle (few KV heads over few tokens), the fp32 sums of
- *   the dk2 / dv2 pass's walk pieces ([pieces <= 8][tokens][heads_kv]
- *   [max(head_dim, value_dim)]). */
+ *   head) work leaves CUs idle (few KV heads over few tokens), room for the sums
+ *   of walk pieces ([up to 8][tokens][heads_kv][max(head_dim, value_dim)]).
+ * The dk2 / dv2 pass cuts its walks into as many pieces, up to 16, as pay and fit
+ * the partials' and the pieces' space together ([head_dim + value_dim] fp32 sums
+ * per piece, token and KV head). */
 size_t sa_prefill_bwd_workspace_bytes(const sa_prefill_bwd_args* args);
 
-/* Backward of sa_prefill_fwd: writes dq, dk1, dk2, dv1, dv2 (each exactly
- * once, fixed reduction order: bitwise reproducible). */
+/* Backward of sa_prefill_fwd: writes dq, dk1, dk2, dv1, dv2 (fixed reduction
+ * order: bitwise reproducible).
+ * Infinite and NaN inputs: the portable kernels touch visible (query, key) pairs
+ * only.  The matrix-core passes multiply the masked entries of a tile by zero, so
+ * that a non-finite value of one token can become NaN in gradients that do not
+ * depend on it, of tokens nearby, of another packed sequence too: dq, dk1 and dv1
+ * of queries and keys that share a tile of 32-35 keys or a workgroup's 1-16
+ * queries with it, dk2 and dv2 of the 32-key groups that its long window overlaps
+ * (and with short windows of at most 16, of the one to three queries next to it in
+ * a step). */
 int sa_prefill_bwd(const sa_prefill_bwd_args* args, void* workspace, size_t workspace_bytes,
                    sa_stream_t stream);
 

@@ -226,16 +226,16 @@ def simplicial_attention(q, k1, k2, v1, v2, short_window, long_window, *, scale=
     [B,N,HQ,DV] in q's dtype and, with ``return_lse=True``, also the
     natural-log LSE [B,N,HQ] in float32.  ``kernel`` selects the
     implementation: "auto" (bf16 with D == DV in {64,128,256}, or with
-    (D, DV) = (128, 64) / (256, 128) as the determinant expansion produces,
+    (D, DV) = (128, 64) / (256, 128) / (512, 256) as the determinant expansion produces,
     and fp32 with D == DV in {64, 128} run on the MFMA kernel; widths 16 and
     32 are zero-padded to 64 to run there too; everything else on the
     portable kernel), "mfma" (raise if not covered) or "generic".
 
     Inputs that require grad get gradients from the library's backward
     (``sa_prefill_bwd``: atomics-free, bitwise reproducible; MFMA tiles for
-    bf16 with D and DV each 64 or 128, or D = 256 over DV = 128 / 256,
-    portable kernels otherwise and with
-    ``kernel="generic"``).  Deviation from
+    bf16 with D and DV each 64 or 128, D = 256 over DV = 128 / 256 or D = 512 over
+    256 with at most 32 short keys, and fp32 with D = DV in {64, 128} and at most
+    32; portable kernels otherwise and with ``kernel="generic"``).  Deviation from
     the reference: forward and backward are deterministic, so
     ``torch.use_deterministic_algorithms(True)`` is allowed.
     """

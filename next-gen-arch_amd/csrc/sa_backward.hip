@@ -588,9 +588,11 @@ static size_t dv1_partial_bytes(const sa_prefill_bwd_args* a) {
   return k + v <= kDk1PartialCap ? v : 0;
 }
 // Scratch for the walk pieces of the dk2 / dv2 pass, beside the partials above
-// (whose space the pieces also take, once they are summed).  Two rules of
-// thumb of the shape: room for the sums of a second row-group's worth of
-// queries where the short window is long for the widths, ...
+// (whose space the pieces also take, once they are summed).  The two rules are
+// those of the dk2 / dv2 kernels before this pass and are kept so that the
+// workspace of a call stays the size it was; how many pieces are taken within it
+// is dkv2_pieces' choice.  One [D + DV] sum where the short window is long for the
+// widths (their second launch), ...
 static size_t dkv2_long_bytes(const sa_prefill_bwd_args* a) {
   const sa_prefill_args& f = a->fwd;
   const bool narrow = (f.head_dim == 64 || f.head_dim == 128) && (f.value_dim == 64 || f.value_dim == 128);
@@ -602,8 +604,8 @@ static size_t dkv2_long_bytes(const sa_prefill_bwd_args* a) {
   return ((size_t)f.total_tokens * f.heads_kv * (f.head_dim + f.value_dim) * sizeof(float) + 255) & ~(size_t)255;
 }
 // ... and, at widths 64 / 128 with short windows of at most 64 keys, up to
-// eight sums of max(D, DV) where 128-key (256-key, widths of 128 that fill the
-// CUs with them) blocks leave the CUs' two workgroup slots empty.
+// eight sums of max(D, DV) where their 128-key (256-key, widths of 128 that fill
+// the CUs with them) workgroups left slots empty, by the LDS that they took.
 static size_t dkv2_split_bytes(const sa_prefill_bwd_args* a) {
   const sa_prefill_args& f = a->fwd;
   const int d = f.head_dim, dv = f.value_dim, cus = device_cu_count();

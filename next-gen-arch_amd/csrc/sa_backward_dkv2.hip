@@ -22,8 +22,12 @@
 // 8 / 2 heads, width 128, windows 32 x 512) bf16 8.39 -> 7.66 ms, fp32 18.96 ->
 // 17.01 ms; width 256, windows 64 x 256, 8192 tokens 12.03 -> 9.69 ms; 16 short
 // keys (2 x 4099 tokens, 16 / 4 heads, 16 x 512) 8.62 -> 7.06 ms.  What bounds
-// it now: one wave per SIMD issues at most one instruction every four cycles,
-// and a step's ~700 (64 of them MFMAs) take longer than its matrix work.
+// it now (counters, adapter shape in bf16): one wave per SIMD, whose chain nothing
+// hides.  It issues in half of its cycles (a step is 535 vector, 64 matrix, 76 LDS
+// and 123 scalar instructions), waits in 38 % -- on the step's barrier and on reloads
+// of spilled values (60 bytes a lane), which in the staging wave wait for the DMA
+// that it has just issued too -- and the matrix cores are busy in 31 %.  fp32 (no
+// spills): 45, 39 and 38 %.
 //
 // Score width 512 (determinant form of 256-wide heads): the accumulators of
 // 512 + 256 columns do not fit; one launch takes dV2 and 128 columns of dK2, a

@@ -17,15 +17,17 @@
 //
 // Measured, forward + backward of the determinant form of 256-wide heads (score
 // width 512, values 256; 1024 tokens, 8 / 2 heads, windows 32 x 256): 271 ms on
-// the portable kernels, 1.8 ms with this pass (0.8 ms in its two column
-// slices) and the dk2 / dv2 pass (0.7 ms).  What bounds it there: LDS, one 1 KB
-// fragment per MFMA, and one wave per SIMD.
+// the portable kernels, 1.70 ms with this pass (0.65 ms in its two column
+// slices) and the dk2 / dv2 pass (0.71 ms).  What bounds it there (counters): the
+// single wave per SIMD waits in 49 % of its cycles, at the start for one load after
+// another of its A and B rows, at the end for one LDS read after another of the
+// sums, and nothing runs beside them; matrix cores busy in 19-20 %.
 // At widths of 64 and 128 with at most 16 short keys it takes the place of the
 // dq pass with dk1 partials and the dv1 pass, whose 32-row tiles such windows
 // half fill: 2 x 4099 tokens, 16 / 4 heads, width 128, 16 x 512 keys 7.06 ->
-// 5.71 ms forward + backward, error against 64 bits 0.0044 before and after.
-// Its partials take less than the scratch that the dk1 partials had.  Two sets
-// of 128 + 128 columns spill 73 registers, outside the unmasked steps.
+// 5.08 ms forward + backward, error against 64 bits 0.0044 before and after
+// (waits 37 %, matrix cores 30 %).  Its partials take less than the scratch that
+// the dk1 partials had.
 //
 // Partials past the workspace: the blocks run in phases (dq_phase), each
 // followed by the sum of the keys it completes; a phase starts with the blocks of

@@ -10,10 +10,11 @@
 //   3  av[c] += Vt^T · P[c]     with dS[c] = P (dP dpm + dsm)
 //   4  ak[c] += Kt^T · dS[c]    with the caller's next-step work
 //
-// What bounds it: every MFMA takes one 1 KB operand fragment from LDS, which
-// at one fragment per MFMA asks for 128 B per cycle and CU -- all that LDS
-// delivers -- before the tile is even written.  With SETS = 2 each fragment
-// feeds two MFMAs.  The accumulators of both gradients and both sets take the
+// Why sets: every MFMA takes one 1 KB operand fragment from LDS, which at one
+// fragment per MFMA asks for 128 B per cycle and CU -- all that LDS delivers --
+// at the full matrix rate.  With SETS = 2 each fragment feeds two MFMAs.  (At the
+// rates reached LDS is not the bound: active in 10-24 % of the cycles, matrix cores
+// in 19-38 %.)  The accumulators of both gradients and both sets take the
 // accumulation registers, so one wave runs per SIMD; the vector work of a
 // phase is therefore placed between the MFMAs of the phase that does not need
 // its result (P beside the dP products, dS beside the av products), one group

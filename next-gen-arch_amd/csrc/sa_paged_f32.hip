@@ -14,9 +14,11 @@
 // Every row keeps its own running maximum; rows, splits and row groups merge
 // by their log-sum-exp weights (paged_combine_kernel, a fixed order).
 //
-// What bounds it: the fp32 matrix rate (a chunk is 128 MFMAs of 64 cycles at
-// width 128, against 32 KB of rows), and for a few tokens the chain of table,
-// rows, products and merge.  So the long axis is cut into as many splits as
+// What bounds it: with many tokens the fp32 matrix rate (a chunk is 128 MFMAs of
+// 64 cycles at width 128, against 32 KB of rows); for a few tokens the chain of
+// rows, products and merge, a tile segment after another since its loads are not
+// issued ahead (the decode below: matrix cores busy in 18 % of the cycles, waves
+// waiting in 48 %).  So the long axis is cut into as many splits as
 // give each SIMD one to four waves.  4 rows x 8 KV heads, GQA 4, 16 x 1025 keys,
 // width 128: 1630 us on the portable kernel (one workgroup per query head, scalar
 // products), 46 us here, of which the merge is 4.

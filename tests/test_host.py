@@ -384,8 +384,8 @@ def test_backward_workspace_reserves_dk1_partials_for_fused_shapes(dtype, hq, hk
     per_query = hq // (4 // nq) * nr * (31 + nq) * d * 4 / nq  # partial bytes per query
     rows = (tokens * hq * 4 + 255) // 256 * 256
     part = (-(-tokens // nq) * (hq // (4 // nq)) * nr * (31 + nq) * d * 4 + 255) // 256 * 256 if fused else 0
-    # short windows of 65-128 at widths <= 128 (33-64 at score width 256): the
-    # fp32 dk2 / dv2 sums of the first of two launches
+    # short windows of 65-128 at widths <= 128 (33-64 at score width 256): one
+    # fp32 dk2 / dv2 sum
     one = 32 if d == 256 else 64
     widths = (d in (64, 128) and dv in (64, 128)) or (d == 256 and dv in (128, 256))
     phased = dtype == "bf16" and widths and one < ws <= 2 * one
@@ -429,14 +429,13 @@ def _dkv2_lds(d, dv, nr, nwk):
 
 
 def _walk_split_bytes(dtype, tokens, hk, d, dv, ws, wl, cus=256):
-    """Workspace of the dk2 / dv2 walk splits (bf16, widths 64 / 128, short
-    window <= 64): when the (key block, KV head) workgroups -- 256 keys (8 waves)
-    if both widths are 128 and they make at least 2 (one group of 32 short rows)
-    or 1 (two groups) per CU, else 128 keys (4 waves) -- number fewer than the
-    CUs' resident slots (two waves per SIMD, or what 160 KB of LDS holds), each
-    walk over the queries is cut into pieces (up to 8, >= 128 queries each),
-    whose fp32 sums take [splits][tokens][hk][max(d, dv)].  Without a GPU the
-    library counts 256 CUs."""
+    """Workspace beside the partials for the pieces of the dk2 / dv2 walks (bf16,
+    widths 64 / 128, short window <= 64), a rule of the shape: where workgroups
+    of 256 keys (both widths 128 and at least 2, with two row groups 1, per CU),
+    else of 128 keys, number fewer than two per CU, or than 160 KB hold of the
+    LDS below, up to 8 sums of [tokens][hk][max(d, dv)] fp32, one per 128 queries
+    of a walk.  (The pass chooses its pieces within the space there is.)  Without
+    a GPU the library counts 256 CUs."""
     if dtype != "bf16" or d not in (64, 128) or dv not in (64, 128) or ws > 64:
         return 0
     nr = 1 if ws <= 32 else 2
