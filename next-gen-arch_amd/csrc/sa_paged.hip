@@ -20,6 +20,7 @@
 // run-to-run bit-identical.
 #include "sa_generic.h"
 #include "sa_mfma.h"
+#include "sa_grid.h"
 #include "sa_launch.h"
 
 namespace sa {
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(const float* __restr
 hipError_t launch_paged_combine(const float* part_o, const float* part_m, const float* part_z, int P,
                                 const sa_paged_args* a, hipStream_t stream) {
   const int64_t nth = (int64_t)a->tokens * a->heads_q;
-  const bool four = P >= 8;
+  const bool four = combine_waves(P, nth) == 4;
   hipLaunchKernelGGL(four ? paged_combine_kernel<4> : paged_combine_kernel<1>,
                      dim3((unsigned)(four ? nth : (nth + 3) / 4)), dim3(256), 0, stream, part_o, part_m, part_z, P,
                      a->tokens, a->heads_q, a->head_dim, a->out, a->o_stride_t, a->o_stride_h, a->lse);

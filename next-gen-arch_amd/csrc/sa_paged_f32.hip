@@ -23,6 +23,7 @@
 // width 128: 1630 us on the portable kernel (one workgroup per query head, scalar
 // products), 46 us here, of which the merge is 4.
 #include "sa_generic.h"
+#include "sa_grid.h"
 #include "sa_mfma.h"
 #include "sa_launch.h"
 
@@ -288,6 +289,7 @@ bool paged_f32_route(const sa_paged_args* a) {
   if ((a->q_stride_t % 4) || (a->q_stride_h % 4)) return false;
   if (((uintptr_t)a->q | (uintptr_t)a->short_cache | (uintptr_t)a->long_cache) & 15) return false;
   const F32Plan f = f32_plan(a);
+  if (!grid_fits((int64_t)a->tokens * a->heads_kv * ((f.tasks + f.nw - 1) / f.nw), 64 * f.nw)) return false;
   return f.nr == 1 || f32_partial_bytes(a, f.nr) <= kF32PartialCap;
 }
 

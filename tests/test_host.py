@@ -311,6 +311,28 @@ def test_paged_plan_bounds_a_global_short_window():
     assert ws <= splits * 16 * 4 * 32 * 130 * 4 + 3 * 256, ws
 
 
+def test_split_merge_grid_holds_every_row(tmp_path):
+    """The merge of 8 partials and more takes a workgroup per (token, head) only
+    where a grid dimension (fewer than 2^32 threads) holds them (csrc/sa_grid.h)."""
+    src, exe = tmp_path / "grid.cpp", tmp_path / "grid"
+    src.write_text("""#include "sa_grid.h"
+#include <cstdio>
+int main() {
+  for (int P : {1, 7, 8, 64})
+    for (long long rows = 1; rows < (1LL << 26); rows = rows * 2 + rows % 3) {
+      const int w = sa::combine_waves(P, rows);
+      const long long threads = (w == 4 ? rows : (rows + 3) / 4) * 256;
+      if (threads >= (1LL << 32) || (w == 4) != (P >= 8 && rows * 256 < (1LL << 32))) return printf("%d %lld\\n", P, rows), 1;
+    }
+  return sa::grid_fits((1LL << 26) - 1, 64) && !sa::grid_fits(1LL << 26, 64) ? 0 : 1;
+}
+""")
+    csrc = os.path.join(ROOT, "next-gen-arch_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-include", "initializer_list", "-I", csrc, str(src), "-o", str(exe)], check=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert run.returncode == 0, run.stdout
+
+
 @pytest.mark.parametrize("short_window", [16, 40])
 def test_fp32_paged_calls_take_any_workspace(short_window):
     """An fp32 query over fp32 caches needed no workspace on the portable kernel:
