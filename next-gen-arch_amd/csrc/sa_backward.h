@@ -68,6 +68,8 @@ hipError_t launch_bwd_dq_core(const BwdParams& p, size_t scratch_bytes, hipStrea
 size_t dq_core_partial_bytes(int tokens, int hq, int hk, int d, int dv, int ws);
 // scratch_bytes: the space at p.dkv2s
 hipError_t launch_bwd_dkv2_mfma(const BwdParams& p, size_t scratch_bytes, hipStream_t stream);
+// ... its fp32 calls and score widths 256 and 512, checked by the former
+hipError_t launch_bwd_dkv2_wide(const BwdParams& p, size_t scratch_bytes, hipStream_t stream);
 // The dq pass can produce dk1 (p.dk1p set): the MFMA passes apply and the
 // short window fits two 32-row groups (one for fp32 inputs).  The MFMA dkv1
 // launch then computes dv1 only.

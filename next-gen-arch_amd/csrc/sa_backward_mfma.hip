@@ -22,7 +22,7 @@
 //     S^T, dP^T, dS as above (A rows q_t ⊙ k1_j, B rows dout_t ⊙ v1_j)
 //     G^T  += K2^T · dS^T,  O''^T += V2^T · bf16(P)^T     (d x t)
 //     dk1_j = Σ_h Σ_t G_t ⊙ q_t,   dv1_j = Σ_h Σ_t O''_t ⊙ dout_t
-//   dk2/dv2 pass: sa_backward_dkv2.hip
+//   dk2/dv2 pass: sa_bwd_dkv2.h
 //
 // The tile machinery (LDS ring filled by global->LDS DMA, TileGeom layouts,
 // the transposing-read accumulation) is the forward kernel's (sa_mfma.h).

@@ -33,6 +33,12 @@ pytestmark = pytest.mark.gpu
     (200, 4, 2, 64, 32, 70, "f32"),
     (131, 4, 2, 64, 8, 40, "f32"),
     (257, 129, 129, 64, 32, 40, "f32"),  # ... 256-key blocks past that
+    # bf16 as well: the shapes above take 128-key blocks, grids that fill the CUs 256-key ones
+    (257, 100, 100, 128, 16, 40, "bf16"),
+    (257, 200, 100, 64, 8, 40, "bf16"),
+    (259, 100, 100, 128, 32, 300, "bf16"),
+    (300, 128, 128, 64, 100, 120, "bf16"),
+    (513, 80, 80, 128, 40, 60, "bf16"),
 ])
 def test_dkv2_step_edges(cuda, n, hq, hk, d, ws, wl, dtype):
     from archlab_amd import simplicial_varlen_attention
