@@ -59,13 +59,15 @@ __device__ __forceinline__ int64_t clamp64(int64_t x, int64_t lo, int64_t hi) { 
 __device__ __forceinline__ int64_t block_of(const void* table, int is64, int64_t row_stride, int width, int64_t nblocks,
                                             int64_t seq, int pos, int block_size) {
   const int64_t col = clamp64(pos / block_size, 0, width - 1);
-  if (table == nullptr) return clamp64(seq * row_stride + col, 0, nblocks - 1);  // consecutive blocks
   return clamp64(load_index(table, seq * row_stride + col, is64), 0, nblocks - 1);
 }
 
 // Paged caches [2 (K,V), blocks, block_size, heads_kv, D] with arbitrary
 // strides.  block = table[seq, pos / block_size] widened to int64 before the
 // stride multiply, slot = pos % block_size (simplicial_paged.py:41-44, :49-52).
+// CONSECUTIVE: blocks of one row at seq * row_stride + position (no tables).  A
+// type of its own: the portable kernel forms an offset per element, and a choice
+// there takes 5-7 % of its time.
 struct PagedRows {
   const void* sc;
   const void* lc;
@@ -79,15 +81,28 @@ struct PagedRows {
   int st_w, lt_w;
   int64_t s_blocks, l_blocks;
   int64_t seq;
-  int s_shift;  // positions before the first short row (consecutive rows; 0 with tables)
+  int s_shift;  // positions before the first short row (consecutive rows)
+};
+
+template <bool CONSECUTIVE>
+struct PagedRowsOf : PagedRows {
   __device__ int64_t s_off(int pos, int g) const {
-    if (s_shift) pos = max(pos - s_shift, 0);
-    const int64_t blk = block_of(stable, stab64, st_s, st_w, s_blocks, seq, pos, block_size);
-    return blk * sc_b + (int64_t)(pos % block_size) * sc_s + (int64_t)g * sc_h;
+    if constexpr (CONSECUTIVE) {
+      const int64_t col = clamp64(pos - s_shift, 0, st_w - 1);
+      return clamp64(seq * st_s + col, 0, s_blocks - 1) * sc_b + (int64_t)g * sc_h;
+    } else {
+      const int64_t blk = block_of(stable, stab64, st_s, st_w, s_blocks, seq, pos, block_size);
+      return blk * sc_b + (int64_t)(pos % block_size) * sc_s + (int64_t)g * sc_h;
+    }
   }
   __device__ int64_t l_off(int pos, int g) const {
-    const int64_t blk = block_of(ltable, ltab64, lt_s, lt_w, l_blocks, seq, pos, block_size);
-    return blk * lc_b + (int64_t)(pos % block_size) * lc_s + (int64_t)g * lc_h;
+    if constexpr (CONSECUTIVE) {
+      const int64_t col = clamp64(pos, 0, lt_w - 1);
+      return clamp64(seq * lt_s + col, 0, l_blocks - 1) * lc_b + (int64_t)g * lc_h;
+    } else {
+      const int64_t blk = block_of(ltable, ltab64, lt_s, lt_w, l_blocks, seq, pos, block_size);
+      return blk * lc_b + (int64_t)(pos % block_size) * lc_s + (int64_t)g * lc_h;
+    }
   }
   __device__ int64_t k1_off(int pos, int g) const { return s_off(pos, g); }
   __device__ int64_t v1_off(int pos, int g) const { return s_off(pos, g) + sc_a; }

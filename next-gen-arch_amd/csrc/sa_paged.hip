@@ -509,12 +509,12 @@ struct GenericPagedParams {
   int hq;
 };
 
-template <typename QT, typename SCT, typename LCT>
+template <typename QT, typename SCT, typename LCT, bool CONSECUTIVE>
 __global__ __launch_bounds__(kGenThreads) void paged_generic_kernel(GenericPagedParams gp) {
   const int token = bid_x(), h = bid_y();
-  PagedRows rows = gp.rows;
-  rows.seq = gp.tseq ? clamp64(load_index(gp.tseq, token, gp.seq64), 0, gp.num_seqs - 1) : token;
-  const int pos = gp.tpos ? (int)load_index(gp.tpos, token, gp.pos64) : gp.wl - 1;
+  PagedRowsOf<CONSECUTIVE> rows{gp.rows};
+  rows.seq = CONSECUTIVE ? token : clamp64(load_index(gp.tseq, token, gp.seq64), 0, gp.num_seqs - 1);
+  const int pos = CONSECUTIVE ? gp.wl - 1 : (int)load_index(gp.tpos, token, gp.pos64);
   int ws = gp.ws, wl = gp.wl;
   if (gp.caps) {
     ws = max(1, min(ws, gp.caps[2 * token]));
@@ -657,7 +657,8 @@ static hipError_t launch_paged_mfma_d(const PagedParams& p, int nw, hipStream_t 
 template <typename QT, typename SCT, typename LCT>
 static hipError_t launch_paged_generic_t(const GenericPagedParams& gp, const sa_paged_args* a, size_t lds,
                                          hipStream_t stream) {
-  auto kern = paged_generic_kernel<QT, SCT, LCT>;
+  auto kern = a->flags & SA_FLAG_CONSECUTIVE_ROWS ? paged_generic_kernel<QT, SCT, LCT, true>
+                                                  : paged_generic_kernel<QT, SCT, LCT, false>;
   hipError_t e = set_lds_limit((const void*)kern, lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3(a->tokens, a->heads_q), dim3(kGenThreads), lds, stream, gp);

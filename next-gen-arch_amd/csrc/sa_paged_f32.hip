@@ -85,7 +85,8 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_f32_kernel(PagedF
   b /= p.splits;
   const int g = b % p.hk, token = b / p.hk;
 
-  PagedRows rows = p.rows;
+  const bool tables = p.rows.stable != nullptr;  // (uniform)
+  PagedRowsOf<false> rows{p.rows};
   rows.seq = p.tseq ? clamp64(load_index(p.tseq, token, p.seq64), 0, p.num_seqs - 1) : token;
   const int pos = p.tpos ? (int)load_index(p.tpos, token, p.pos64) : p.wl - 1;
   int ws = p.ws, wl = p.wl;
@@ -109,7 +110,11 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_f32_kernel(PagedF
   const int h = g * p.group + (head_ok ? hi : 0);
   const SCT* const sc = (const SCT*)rows.sc;
   const LCT* const lc = (const LCT*)rows.lc;
-  const int64_t soff = rows.s_off(max(j, 0), g);
+  auto at = [&](auto off) {  // off(rows) of the caches' form
+    PagedRowsOf<true> seq_rows{rows};
+    return tables ? off(rows) : off(seq_rows);
+  };
+  const int64_t soff = at([&](const auto& x) { return x.s_off(max(j, 0), g); });
 
   floatx4 a[D / 8];  // A rows: d = 8 u + 4 half + e; during the last P·V the v1 rows
   floatx16 o[D / 32];
@@ -120,7 +125,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_f32_kernel(PagedF
   for (int c = cbeg; c < cend; ++c) {
     const int k0 = kstart + kChunk * c;
     __syncthreads();  // the previous chunk is consumed
-    if (tid < kChunk) roff[tid] = rows.l_off(min(max(k0 + tid, lo2), pos), g);
+    if (tid < kChunk) roff[tid] = at([&](const auto& x) { return x.l_off(min(max(k0 + tid, lo2), pos), g); });
     __syncthreads();
     if (c == cbeg) {  // beside the first tile's loads
       const float* const qr = p.q + (int64_t)token * p.q_st + (int64_t)h * p.q_sh;
